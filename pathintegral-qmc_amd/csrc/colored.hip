@@ -31,6 +31,7 @@
 #include <type_traits>
 
 #include "piqmc_internal.h"
+#include "sparse.h"
 
 namespace {
 
@@ -2503,11 +2504,36 @@ size_t colored_scratch_bytes(const piqmc_problem *pb, int R, int P, int S)
     return b + CallBuffers::round_up(wb * 2 * (size_t)pb->N * R);
 }
 
+// Tile of the sparse real-coupling sweep (block 0: it does not apply).  The
+// caller's block and rpw are kept; by default a workgroup has the lanes that
+// take a slot's words (two color classes) in whole passes of at most 1024.
+struct SparseTile {
+    int block, rpw;
+};
+SparseTile sparse_tile(const piqmc_problem *pb, int R, size_t word_bytes, int block, int rpw, bool chains)
+{
+    if (!pb->sparse_rows || block > 1024 || (block > 0 && (block & 63)) || rpw > 64) return {0, 0};
+    if (rpw <= 0) rpw = 1;
+    if (block <= 0) {
+        int most = 0;
+        for (int c = 0; c < pb->ncolors; ++c) {
+            const int n0 = pb->color_off[c + 1] - pb->color_off[c];
+            const int c1 = c ? c - 1 : pb->ncolors - 1;
+            const int n1 = chains || c1 == c ? 0 : pb->color_off[c1 + 1] - pb->color_off[c1];
+            most = std::max(most, ((n0 + 63) & ~63) + n1);
+        }
+        const int passes = (most + 1023) / 1024;
+        block = ((most + passes - 1) / passes + 63) & ~63;
+    }
+    if (piqmc::sparse_lds(pb->N, rpw, (int)word_bytes, block) > 160 * 1024) return {0, 0};
+    return {block, rpw};
+}
+
 template <typename WT>
 int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
                 const std::vector<float> &jp, const std::vector<float> &temps, int8_t *confs, uint64_t seed, uint32_t rbase,
                 uint32_t sbase, double *etrace, int block, int rpw, hipStream_t st,
-                unsigned char *scratch = nullptr, size_t scratch_cap = 0)
+                unsigned char *scratch = nullptr, size_t scratch_cap = 0, bool chains = false)
 {
     const int N = pb->N;
     CallBuffers buf;
@@ -2624,6 +2650,11 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
     }
     std::vector<uint32_t> thr, ztab;
     const bool pmj = pb->pmj && pmj_tables(pb, S, jp, temps, thr, ztab);
+    // real couplings with short rows: the filtered sweep of sparse.hip, where
+    // its planes and queues fit the LDS; longer rows and larger planes keep the
+    // per-bit general path
+    const SparseTile tile = sparse_tile(pb, R, sizeof(WT), block, rpw, chains);
+    const bool sparse = tile.block > 0;
     if (rpw <= 0 && pb->pmjf && !pb->pmj && pb->ncolors == 2 && pb->zuni_nf == 6 && cached_fields_enabled()) {
         // the cached field sweep evaluates each step's decision classes once per
         // workgroup for all of its replicas: as many replicas per workgroup as
@@ -2644,11 +2675,12 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         rpw = kFixRep;
         block = (int)kFixBlock;
     }
-    if (rpw <= 0) rpw = R >= 2048 ? 4 : (R >= 1024 ? 2 : 1);
+    if (rpw <= 0) rpw = sparse ? tile.rpw : (R >= 2048 ? 4 : (R >= 1024 ? 2 : 1));
     if (rpw > 64) return piqmc::set_error(PIQMC_EINVAL, "replicas per workgroup must be <= 64");
     const size_t lds = sizeof(WT) * 2 * (size_t)N * rpw + 4 * (kClassStride + 8) + 16 * sizeof(double);
     if (lds > 160 * 1024)
         return piqmc::set_error(PIQMC_EINVAL, "colored sweep: replicas per workgroup x 2 x nspins x P/2 bits exceed one workgroup's LDS");
+    if (block <= 0 && sparse) block = tile.block;
     if (block <= 0) {
         // 256 threads; 512 when a color class would take more than two passes
         // of 256 (measured on the 1728-spin 3-D lattice: 1.08e12 vs 0.84e12
@@ -2691,7 +2723,11 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
     a.packed = d_packed; a.etrace = etrace;
     const int grid = (R + rpw - 1) / rpw;
     piqmc::timing_begin(st);
-    if (!pmj && pb->pmjf) {
+    if (sparse) {
+        const piqmc::SparseCall c = {pb, R, P, S, M, rpw, block, chains, seed, rbase, sbase, d_jp, d_jp + S, d_coff,
+                                     d_packed, etrace};
+        if ((rc = piqmc::sparse_launch(c, st))) return rc;
+    } else if (!pmj && pb->pmjf) {
         a.zuni = -1;
         int biggest = 0;
         for (int c = 0; c < pb->ncolors; ++c) biggest = std::max(biggest, pb->color_off[c + 1] - pb->color_off[c]);
@@ -2849,7 +2885,7 @@ extern "C" int piqmc_sa_colored(const piqmc_problem *pb, int C, int S, int M, co
     }
     hipStream_t st = (hipStream_t)stream;
     return run_colored<uint32_t>(pb, C / P, P, S, M, jp, temps, spins, seed, rbase, sbase, nullptr, block,
-                                 rpw, st);
+                                 rpw, st, nullptr, 0, true);
 }
 
 #include "batch_part.inc"

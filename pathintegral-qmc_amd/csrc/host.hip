@@ -15,6 +15,7 @@
 #include <tuple>
 #include <cstring>
 #include "piqmc_internal.h"
+#include "sparse.h"
 
 namespace piqmc {
 static thread_local std::string g_err;
@@ -274,6 +275,10 @@ static int upload_coloring(piqmc_problem &p)
     }
     PIQMC_HIP(hipMalloc(&p.d_prevj, sizeof(double) * N));
     PIQMC_HIP(hipMemcpy(p.d_prevj, prevj.data(), sizeof(double) * N, hipMemcpyHostToDevice));
+    if (!p.pmj && !p.pmjf) {
+        const int rc = piqmc::sparse_upload(p, order);
+        if (rc) return rc;
+    }
     if (p.pmj || p.pmjf) {
         const int zm = std::max(p.zmax, 1);
         std::vector<int32_t> cnb((size_t)zm * N, 0);
@@ -484,6 +489,7 @@ extern "C" int piqmc_problem_create_dense(int N, const double *Jm, int64_t s0, i
 extern "C" int piqmc_problem_destroy(piqmc_problem *p)
 {
     if (!p) return PIQMC_OK;
+    piqmc::sparse_free(*p);
     if (p->d_rows) (void)hipFree(p->d_rows);
     if (p->d_jd) (void)hipFree(p->d_jd);
     if (p->d_order) (void)hipFree(p->d_order);

@@ -26,6 +26,21 @@ int check_perms(const uint16_t *perms, size_t n, int N, hipStream_t st);
     } while (0)
 
 // ------------------------------------------------------------------ problem
+namespace piqmc {
+// Tables of the sparse real-coupling sweep by color position q: the row's
+// nonzero couplings in row order, padded to `sparse_rows` entries; the arrays
+// over entries have 8 places a row for 6 entries (sparse.hip builds and reads
+// them).
+constexpr int kSparseMaxRow = 16, kSparsePlanes = 8;
+struct SparseTab {
+    const uint16_t *nb = nullptr;  // [N][places] neighbour, N for a field and for padding
+    const float *J = nullptr;      // [N][places] coupling, 0 for padding
+    const uint32_t *w = nullptr;   // [N][places/4] |J| as 8-bit weights, four to a word
+    const uint4 *meta = nullptr;   // [N] spin | (bit z: J < 0) << 16, and three floats:
+                                   // weight per unit of |J|, the base of the accept and
+                                   // of the reject threshold
+};
+}  // namespace piqmc
 // A neighbour table (tools.GenerateNeighbors format) resident in HBM, with the
 // analysis the colored sweep needs.
 struct piqmc_problem {
@@ -69,6 +84,11 @@ struct piqmc_problem {
     // [N] sum of the couplings of spin order[q] to spin order[q-1] (0 at q = 0):
     // the pipelined dense sweep adds that neighbour's term after its decision
     double *d_prevj = nullptr;
+    // Real couplings with short rows: entries per row (4, 6, 8 or 16; 0 when
+    // the problem has no such tables).
+    piqmc::SparseTab sparse;
+    int sparse_rows = 0;
+    unsigned char *d_sparse = nullptr;  // what the tables' arrays are parts of
 };
 
 // ------------------------------------------------------------------ device helpers
