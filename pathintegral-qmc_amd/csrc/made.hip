@@ -347,23 +347,24 @@ __global__ __launch_bounds__(256) void gemm_nt_bf16_tile(const uint16_t *A, int 
 // groups' partial tiles meet in LDS and are summed in group order (the result
 // does not depend on timing).  Loads past the last stage repeat it, so every
 // group issues the same loads; stages past the end are not computed.
+constexpr int kRedPitch = GT + 4;  // floats per row of a partial tile
 template <int KG>
-__global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_splitk(const uint16_t *A, int lda, const uint16_t *B,
-                                                              int ldb, int M, int N, int K, const float *bias,
-                                                              int relu, float *Cf, uint16_t *Cb, int ldc)
+constexpr size_t kSplitLds = (size_t)KG * 4 * GT * PKP * 2 > (size_t)KG * GT * kRedPitch * 4
+                                 ? (size_t)KG * 4 * GT * PKP * 2 : (size_t)KG * GT * kRedPitch * 4;
+
+// The K loop of one tile at (m0, n0): leaves the groups' partial tiles in
+// smem as floats [KG][GT][kRedPitch], behind a barrier.
+template <int KG>
+__device__ __forceinline__ void splitk_tile(const uint16_t *A, int lda, const uint16_t *B, int ldb, int M, int N,
+                                            int K, int m0, int n0, unsigned char *smem)
 {
     constexpr int kBuf = GT * PKP;                        // bf16 per stage buffer of A or of B
-    constexpr int kRedPitch = GT + 4;                     // floats per row of a partial tile
-    constexpr size_t kStageBytes = (size_t)KG * 4 * kBuf * 2;  // per group: A x 2 buffers, B x 2 buffers
-    constexpr size_t kRedBytes = (size_t)KG * GT * kRedPitch * 4;
-    __shared__ __align__(16) unsigned char smem[kStageBytes > kRedBytes ? kStageBytes : kRedBytes];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const int grp = wid >> 2, gt = tid & 255, gw = wid & 3;
     uint16_t *As = reinterpret_cast<uint16_t *>(smem) + (size_t)grp * 4 * kBuf;  // [buf][row][k]
     uint16_t *Bs = As + 2 * kBuf;
     auto a_at = [&](int buf, int r, int k) -> uint16_t * { return As + buf * kBuf + r * PKP + k; };
     auto b_at = [&](int buf, int r, int k) -> uint16_t * { return Bs + buf * kBuf + r * PKP + k; };
-    const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
     const int wm = (gw >> 1) * 32, wn = (gw & 1) * 32;
     f32x4 acc[2][2];
 #pragma unroll
@@ -437,6 +438,17 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_splitk(const uint16_t *
                 red[((size_t)grp * GT + wm + a * 16 + (lane >> 4) * 4 + j) * kRedPitch + wn + b * 16 + (lane & 15)] =
                     acc[a][b][j];
     __syncthreads();
+}
+
+template <int KG>
+__global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_splitk(const uint16_t *A, int lda, const uint16_t *B,
+                                                              int ldb, int M, int N, int K, const float *bias,
+                                                              int relu, float *Cf, uint16_t *Cb, int ldc)
+{
+    __shared__ __align__(16) unsigned char smem[kSplitLds<KG>];
+    const int tid = threadIdx.x, m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
+    splitk_tile<KG>(A, lda, B, ldb, M, N, K, m0, n0, smem);
+    const float *red = reinterpret_cast<const float *>(smem);
     for (int idx = tid; idx < GT * GT; idx += 256 * KG) {
         const int rl = idx / GT, cl = idx % GT, row = m0 + rl, col = n0 + cl;
         if (row < M && col < N) {
@@ -503,31 +515,32 @@ void gemm(const uint16_t *A, int lda, const uint16_t *B, int ldb, int M, int N, 
 }
 
 // ------------------------------------------------------------------ elementwise
-__global__ void spins_to_bf16(const int8_t *s, size_t n, uint16_t *x)
+__global__ void spins_to_bf16(const int8_t *s, int B, int N, uint16_t *x, int ldx)
 {
+    const size_t n = (size_t)B * N;
     for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x)
-        x[t] = s[t] < 0 ? 0xBF80u : 0x3F80u;  // -1.0 / +1.0 in bf16
+        x[t / N * ldx + t % N] = s[t] < 0 ? 0xBF80u : 0x3F80u;  // -1.0 / +1.0 in bf16
 }
 
-// transpose bf16 [R][C] -> [C][R]
-__global__ void transpose_bf16(const uint16_t *in, int R, int C, uint16_t *out)
+// transpose bf16 [R][ldi] -> [C][ldo]
+__global__ void transpose_bf16(const uint16_t *in, int R, int C, int ldi, uint16_t *out, int ldo)
 {
     __shared__ uint16_t tile[32][33];
     const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
     for (int y = threadIdx.y; y < 32; y += blockDim.y) {
         const int r = by + y, c = bx + threadIdx.x;
-        tile[y][threadIdx.x] = (r < R && c < C) ? in[(size_t)r * C + c] : 0;
+        tile[y][threadIdx.x] = (r < R && c < C) ? in[(size_t)r * ldi + c] : 0;
     }
     __syncthreads();
     for (int y = threadIdx.y; y < 32; y += blockDim.y) {
         const int c = bx + y, r = by + threadIdx.x;
-        if (c < C && r < R) out[(size_t)c * R + r] = tile[threadIdx.x][y];
+        if (c < C && r < R) out[(size_t)c * ldo + r] = tile[threadIdx.x][y];
     }
 }
 
 // Output layer loss: per sample nll = sum_d softplus(l_d) - b_d l_d; grad
 // dL/dl (scaled by gscale) to bf16 dlog [B][N]; per-sample nll to out.
-__global__ void output_nll(const float *logits, const int8_t *s, int B, int N, float gscale, uint16_t *dlog,
+__global__ void output_nll(const float *logits, const int8_t *s, int B, int N, float gscale, uint16_t *dlog, int ldd,
                            double *nll, double sign)
 {
     const int b = blockIdx.x;
@@ -539,7 +552,7 @@ __global__ void output_nll(const float *logits, const int8_t *s, int B, int N, f
         acc += sp - (double)bit * (double)l;
         if (dlog) {
             const float sg = 1.f / (1.f + expf(-l));
-            dlog[(size_t)b * N + d] = f2bf_bits((sg - bit) * gscale);
+            dlog[(size_t)b * ldd + d] = f2bf_bits((sg - bit) * gscale);
         }
     }
     __shared__ double red[16];
@@ -566,56 +579,296 @@ __global__ void relu_back(uint16_t *dh, const uint16_t *h, size_t n)
         if (!(bf2f(h[t]) > 0.f)) dh[t] = 0;
 }
 
-// column sums of bf16 [B][C] -> fp32 [C]
-__global__ void col_sum_bf16(const uint16_t *g, int B, int C, float *out)
+// Sums over the batch of one unit's values, in batch order, for 64 units (lanes
+// of the first wavefront), from the transposed gradients gt [C][ld]: one add
+// chain a unit, so its time is the chain's and the loads have to stay ahead of
+// it -- the workgroup brings 256 values a unit to LDS at a time.  (A thread a
+// column reading row after row waited for memory at every row: 234 us for
+// 1024 x 512.)
+constexpr int kSumChunk = 256, kSumPitch = kSumChunk + 8;
+constexpr size_t kSumLds = (size_t)64 * kSumPitch * 2;
+__device__ __forceinline__ float unit_sum(const uint16_t *gt, int ld, int C, int c0, int B, unsigned char *smem)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C) return;
+    uint16_t *t = reinterpret_cast<uint16_t *>(smem);
     float s = 0.f;
-    for (int b = 0; b < B; ++b) s += bf2f(g[(size_t)b * C + c]);
-    out[c] = s;
+    for (int b0 = 0; b0 < B; b0 += kSumChunk) {
+        __syncthreads();
+        // rows are padded to 64 values, the last chunk may be shorter
+        const int n8 = (min(B - b0, kSumChunk) + 7) / 8;
+        for (int x = threadIdx.x; x < 64 * (kSumChunk / 8); x += blockDim.x) {
+            const int r = x / (kSumChunk / 8), k = x % (kSumChunk / 8);
+            if (c0 + r < C && k < n8)
+                *reinterpret_cast<uint4 *>(t + r * kSumPitch + 8 * k) =
+                    *reinterpret_cast<const uint4 *>(gt + (size_t)(c0 + r) * ld + b0 + 8 * k);
+        }
+        __syncthreads();
+        if (threadIdx.x < 64 && c0 + (int)threadIdx.x < C) {
+            const int n = min(B - b0, kSumChunk);
+            const uint16_t *v = t + threadIdx.x * kSumPitch;
+            auto add8 = [&](const uint4 q, int m) __attribute__((always_inline)) {
+                const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (j < m) s += __uint_as_float(j & 1 ? w[j / 2] & 0xffff0000u : w[j / 2] << 16);
+            };
+            int b = 0;
+            for (; b + 64 <= n; b += 64) {  // eight reads in flight ahead of the chain
+                uint4 q[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) q[k] = *reinterpret_cast<const uint4 *>(v + b + 8 * k);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) add8(q[k], 8);
+            }
+            for (; b < n; b += 8) add8(*reinterpret_cast<const uint4 *>(v + b), n - b);
+        }
+    }
+    return s;
 }
 
-// Adam step on fp32 master weights (masked), refresh bf16 W [O][I] and W^T [I][O].
-__global__ void adam_w(float *w, float *m, float *v, const float *g, const uint8_t *mask, int O, int I,
-                       float lr, float b1, float b2, float eps, float c1, float c2, uint16_t *wb, uint16_t *wt)
+__global__ void __launch_bounds__(256) unit_sum_kernel(const uint16_t *gt, int ld, int C, int B, float *out)
+{
+    __shared__ __align__(16) unsigned char smem[kSumLds];
+    const int c0 = blockIdx.x * 64;
+    const float s = unit_sum(gt, ld, C, c0, B, smem);
+    if (threadIdx.x < 64 && c0 + (int)threadIdx.x < C) out[c0 + threadIdx.x] = s;
+}
+
+struct Adam {
+    float lr, b1, b2, eps, c1, c2;
+};
+// One parameter's step from its gradient: moments in place, the new value.
+__device__ __forceinline__ float adam_one(const Adam &h, float w, float *m, float *v, float gr)
+{
+    const float mv = h.b1 * *m + (1.f - h.b1) * gr;
+    const float vv = h.b2 * *v + (1.f - h.b2) * gr * gr;
+    *m = mv;
+    *v = vv;
+    return w - h.lr * (mv / h.c1) / (sqrtf(vv / h.c2) + h.eps);
+}
+
+// Adam step on fp32 master weights (masked), refresh bf16 W [O][ldw] and W^T [I][ldt].
+__global__ void adam_w(float *w, float *m, float *v, const float *g, const uint8_t *mask, int O, int I, Adam h,
+                       uint16_t *wb, int ldw, uint16_t *wt, int ldt)
 {
     const size_t n = (size_t)O * I;
     for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x) {
-        float wv = 0.f;
-        if (mask[t]) {
-            const float gr = g[t];
-            const float mv = b1 * m[t] + (1.f - b1) * gr;
-            const float vv = b2 * v[t] + (1.f - b2) * gr * gr;
-            m[t] = mv;
-            v[t] = vv;
-            wv = w[t] - lr * (mv / c1) / (sqrtf(vv / c2) + eps);
-        }
+        const float wv = mask[t] ? adam_one(h, w[t], m + t, v + t, g[t]) : 0.f;
         w[t] = wv;
         const uint16_t bb = f2bf_bits(wv);
-        wb[t] = bb;
         const int o = (int)(t / I), i = (int)(t % I);
-        wt[(size_t)i * O + o] = bb;
+        wb[(size_t)o * ldw + i] = bb;
+        wt[(size_t)i * ldt + o] = bb;
     }
 }
 
-__global__ void adam_b(float *b, float *m, float *v, const float *g, int n, float lr, float b1, float b2,
-                       float eps, float c1, float c2)
+__global__ void adam_b(float *b, float *m, float *v, const float *g, int n, Adam h)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const float gr = g[t];
-    const float mv = b1 * m[t] + (1.f - b1) * gr;
-    const float vv = b2 * v[t] + (1.f - b2) * gr * gr;
-    m[t] = mv;
-    v[t] = vv;
-    b[t] -= lr * (mv / c1) / (sqrtf(vv / c2) + eps);
+    if (t < n) b[t] = adam_one(h, b[t], m + t, v + t, g[t]);
+}
+
+// ------------------------------------------------------------------ training kernels
+// A training step at the sizes the proposal networks have is a chain of small
+// kernels whose start and end cost more than their work.  So each product's
+// epilogue does what separate passes did (ReLU and its mask, the transposed
+// copy that the weight gradients need, Adam), and the three weight gradients
+// with the bias sums run in one launch: 8 kernels a step instead of 29 (256-512
+// network, batch 1024: 0.80 -> 0.07 ms a step; 5.6-9.6 us a kernel, 15 us the
+// weight gradients, against a launch floor of about 3 us each).  All
+// values are those of the separate passes: the products keep their order of
+// summation (the number of K groups, kg), the rest is elementwise.
+// Row pitches of the bf16 operands are multiples of 64 with zeros past the
+// sizes, so K is rounded up to whole stages and rows are 16-byte aligned.
+struct TrainGemm {
+    const uint16_t *A, *B;
+    int lda, ldb, M, N, K;
+    const float *bias;      // forward
+    int relu;
+    const uint16_t *keep;   // backward: zero where !(keep > 0), pitch ldc
+    float *Cf;              // [M][ldf]
+    int ldf;
+    uint16_t *Cb;           // [M][ldc]
+    int ldc;
+    uint16_t *Ct;           // [N][ldt], zeros for the rows past M of the last tile
+    int ldt;
+    // weight gradients (the kernel of several jobs): Cf is the gradient, then
+    // with step an Adam step of the masters, Cb / Ct the weights and their
+    // transpose
+    int step;
+    float *w, *m, *v;
+    const uint8_t *mask;
+    // bias gradients from Ct-layout gradients gt [units][ldg]: n64 blocks of 64
+    const uint16_t *gt;
+    int ldg, units, rows, n64;
+    float *gb, *b, *bm, *bv;
+};
+template <int NJ>
+struct TrainJobs {
+    TrainGemm j[NJ];
+    int n, blocks[NJ];      // workgroups of each job: its n64 bias blocks first
+    Adam h;
+};
+
+template <int KG, int NJ>
+__global__ __launch_bounds__(256 * KG) void train_gemm(TrainJobs<NJ> jobs)
+{
+    __shared__ __align__(16) unsigned char smem[kSplitLds<KG>];
+    static_assert(kSplitLds<KG> >= kSumLds, "bias sums fit the tile's LDS");
+    int bx = blockIdx.x, jn = 0;
+    if constexpr (NJ > 1)
+        while (jn + 1 < jobs.n && bx >= jobs.blocks[jn]) bx -= jobs.blocks[jn++];
+    const TrainGemm &g = jobs.j[NJ > 1 ? jn : 0];
+    const int tid = threadIdx.x;
+    if constexpr (NJ > 1) {
+        if (bx < g.n64) {
+            const int c = bx * 64 + tid;
+            const float s = unit_sum(g.gt, g.ldg, g.units, bx * 64, g.rows, smem);
+            if (tid < 64 && c < g.units) {
+                g.gb[c] = s;
+                if (g.step) g.b[c] = adam_one(jobs.h, g.b[c], g.bm + c, g.bv + c, s);
+            }
+            return;
+        }
+        bx -= g.n64;
+    }
+    const int tn = (g.N + GT - 1) / GT, m0 = bx / tn * GT, n0 = bx % tn * GT;
+    constexpr int kTrips = GT * GT / (256 * KG);
+    constexpr int kAhead = KG == 4 ? kTrips : 1;  // elements whose Adam state is read before the product
+    float pw[kAhead], pm[kAhead], pv[kAhead];
+    uint8_t pk[kAhead];
+    if constexpr (NJ > 1 && KG == 4) {
+        if (g.step) {
+#pragma unroll
+            for (int k = 0; k < kAhead; ++k) {
+                const int idx = tid + k * 256 * KG, row = min(m0 + idx / GT, g.M - 1), col = min(n0 + idx % GT, g.N - 1);
+                const size_t t = (size_t)row * g.N + col;
+                pk[k] = g.mask[t];
+                pw[k] = g.w[t];
+                pm[k] = g.m[t];
+                pv[k] = g.v[t];
+            }
+        }
+    }
+    splitk_tile<KG>(g.A, g.lda, g.B, g.ldb, g.M, g.N, g.K, m0, n0, smem);
+    float *red = reinterpret_cast<float *>(smem);
+#pragma unroll
+    for (int k = 0; k < kTrips; ++k) {
+        const int idx = tid + k * 256 * KG, rl = idx / GT, cl = idx % GT, row = m0 + rl, col = n0 + cl;
+        uint32_t bits = 0;  // bf16 of the value kept for the transposed copy
+        if (row < g.M && col < g.N) {
+            float v = 0.f;
+#pragma unroll
+            for (int q = 0; q < KG; ++q) v += red[((size_t)q * GT + rl) * kRedPitch + cl];
+            if (g.bias) v += g.bias[col];
+            if (g.relu) v = v > 0.f ? v : 0.f;
+            if (g.Cf) g.Cf[(size_t)row * g.ldf + col] = v;
+            if constexpr (NJ > 1) {
+                if (g.step) {
+                    const size_t t = (size_t)row * g.N + col;
+                    if constexpr (KG == 4) {
+                        if (pk[k]) {
+                            v = adam_one(jobs.h, pw[k], &pm[k], &pv[k], v);
+                            g.m[t] = pm[k];
+                            g.v[t] = pv[k];
+                        } else {
+                            v = 0.f;
+                        }
+                    } else {
+                        v = g.mask[t] ? adam_one(jobs.h, g.w[t], g.m + t, g.v + t, v) : 0.f;
+                    }
+                    g.w[t] = v;
+                }
+            }
+            bits = f2bf_bits(v);
+            if (g.keep && !(bf2f(g.keep[(size_t)row * g.ldc + col]) > 0.f)) bits = 0;
+            if (g.Cb && (NJ == 1 || g.step)) g.Cb[(size_t)row * g.ldc + col] = (uint16_t)bits;
+        }
+        red[(size_t)rl * kRedPitch + cl] = __uint_as_float(bits);  // its own partial sums are read
+    }
+    if (!g.Ct || (NJ > 1 && !g.step)) return;
+    __syncthreads();
+    for (int idx = tid; idx < GT * GT / 8; idx += 256 * KG) {
+        const int cl = idx / 8, rl = (idx % 8) * 8;
+        if (n0 + cl >= g.N) continue;
+        uint32_t q[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            q[j] = __float_as_uint(red[(size_t)(rl + 2 * j) * kRedPitch + cl]) |
+                   (__float_as_uint(red[(size_t)(rl + 2 * j + 1) * kRedPitch + cl]) << 16);
+        *reinterpret_cast<uint4 *>(g.Ct + (size_t)(n0 + cl) * g.ldt + m0 + rl) = make_uint4(q[0], q[1], q[2], q[3]);
+    }
+}
+
+// Rows s[perm[b0 + b]] (perm null: s[b0 + b]) as bf16 spins x [B][ldx] and
+// transposed xt [N][ldt]: 64 x 64 tiles, zeros past row B of xt.
+__global__ void __launch_bounds__(256) train_input(const int8_t *s, const int32_t *perm, int b0, int B, int N,
+                                                   uint16_t *x, int ldx, uint16_t *xt, int ldt)
+{
+    __shared__ uint16_t tile[64][72];
+    const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
+    for (int t = threadIdx.x; t < 64 * 64; t += 256) {
+        const int r = t / 64, c = t % 64, b = r0 + r, i = c0 + c;
+        uint16_t v = 0;
+        if (b < B && i < N) {
+            v = s[(size_t)(perm ? perm[b0 + b] : b0 + b) * N + i] < 0 ? 0xBF80u : 0x3F80u;
+            x[(size_t)b * ldx + i] = v;
+        }
+        tile[c][r] = v;
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < 64 * 8; t += 256) {
+        const int c = t / 8, r = (t % 8) * 8;
+        if (c0 + c < N)
+            *reinterpret_cast<uint4 *>(xt + (size_t)(c0 + c) * ldt + r0 + r) =
+                *reinterpret_cast<const uint4 *>(&tile[c][r]);
+    }
+}
+
+constexpr int kNllRows = 4;
+// output_nll of kNllRows rows a workgroup (more leave CUs idle in the double logarithms) with the gradient's transposed copy
+// dt [N][ldt] (zeros past row B): spins are read from the signs of x.
+__global__ void __launch_bounds__(256) train_nll(const float *logits, const uint16_t *x, int ldx, int B, int N,
+                                                 float gscale, uint16_t *dlog, int ldd, uint16_t *dt, int ldt,
+                                                 double *nll)
+{
+    const int b0 = blockIdx.x * kNllRows;
+    double acc[kNllRows] = {};
+    for (int d = threadIdx.x; d < N; d += 256) {
+        uint32_t q[kNllRows / 2] = {};
+#pragma unroll
+        for (int r = 0; r < kNllRows; ++r) {
+            const int b = b0 + r;
+            if (b >= B) continue;
+            const float l = logits[(size_t)b * N + d];
+            const float bit = (x[(size_t)b * ldx + d] & 0x8000u) ? 1.f : 0.f;
+            const double sp = l > 0 ? (double)l + log1p(exp(-(double)l)) : log1p(exp((double)l));
+            acc[r] += sp - (double)bit * (double)l;
+            const float sg = 1.f / (1.f + expf(-l));
+            const uint32_t g = f2bf_bits((sg - bit) * gscale);
+            dlog[(size_t)b * ldd + d] = (uint16_t)g;
+            q[r / 2] |= g << (16 * (r & 1));
+        }
+        *reinterpret_cast<uint2 *>(dt + (size_t)d * ldt + b0) = make_uint2(q[0], q[1]);
+    }
+    __shared__ double red[kNllRows][4];
+#pragma unroll
+    for (int r = 0; r < kNllRows; ++r) {
+        for (int o = 32; o > 0; o >>= 1) acc[r] += __shfl_xor(acc[r], o, 64);
+        if ((threadIdx.x & 63) == 0) red[r][threadIdx.x >> 6] = acc[r];
+    }
+    __syncthreads();
+    if (threadIdx.x < kNllRows && b0 + (int)threadIdx.x < B) {
+        double t = 0;
+        for (int w = 0; w < 4; ++w) t += red[threadIdx.x][w];
+        nll[b0 + threadIdx.x] = 1.0 * t;
+    }
 }
 
 // Sampling step d: draw s_d for every row from sigmoid(logit d).  The key and
 // round come from device memory (rng = {key0, key1, round}) so that the
 // captured sampling graph stays valid across calls.
-__global__ void sample_step(const float *logits, int B, int N, int d, const uint32_t *rng, int8_t *s, uint16_t *x)
+__global__ void sample_step(const float *logits, int B, int N, int d, const uint32_t *rng, int8_t *s, uint16_t *x,
+                            int ldx)
 {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= B) return;
@@ -626,7 +879,7 @@ __global__ void sample_step(const float *logits, int B, int N, int d, const uint
     const double p = 1.0 / (1.0 + exp(-(double)l));  // p(s_d = -1)
     const bool neg = u < p;
     s[(size_t)b * N + d] = neg ? -1 : 1;
-    x[(size_t)b * N + d] = neg ? 0xBF80u : 0x3F80u;
+    x[(size_t)b * ldx + d] = neg ? 0xBF80u : 0x3F80u;
 }
 
 }  // namespace
@@ -634,46 +887,61 @@ __global__ void sample_step(const float *logits, int B, int N, int d, const uint
 #include "made_state.h"
 
 namespace {
+int up64(int n) { return (n + 63) & ~63; }
+
+// Row pitches of the layers' inputs and of the logits (multiples of 64; what
+// lies past the sizes is zeroed here and never written).
 int made_alloc_batch(piqmc_made *m, int B)
 {
     if (B <= m->cap) return PIQMC_OK;
-    const int N = m->N, H1 = m->H1, H2 = m->H2;
+    const int N = m->N, H1 = m->H1, H2 = m->H2, lN = up64(N), l1 = up64(H1), l2 = up64(H2), lB = up64(B);
     void **bufs[] = {(void **)&m->x, (void **)&m->h1, (void **)&m->h2, (void **)&m->logits, (void **)&m->dlog,
-                     (void **)&m->dh2, (void **)&m->dh1, (void **)&m->tA, (void **)&m->tB, (void **)&m->nll,
-                     (void **)&m->s};
+                     (void **)&m->dh2, (void **)&m->dh1, (void **)&m->xt, (void **)&m->h1t, (void **)&m->h2t,
+                     (void **)&m->dlogt, (void **)&m->dh2t, (void **)&m->dh1t, (void **)&m->nll, (void **)&m->s};
     for (auto p : bufs)
         if (*p) (void)hipFree(*p), *p = nullptr;
+    m->cap = 0;
     if (m->gexec) (void)hipGraphExecDestroy(m->gexec), m->gexec = nullptr, m->gB = 0;  // holds old addresses
-    const int Hm = std::max(std::max(H1, H2), N);
-    PIQMC_HIP(hipMalloc(&m->x, 2 * (size_t)B * N));
-    PIQMC_HIP(hipMalloc(&m->h1, 2 * (size_t)B * H1));
-    PIQMC_HIP(hipMalloc(&m->h2, 2 * (size_t)B * H2));
+    auto zeroed = [](uint16_t **p, size_t n) -> hipError_t {
+        hipError_t e = hipMalloc((void **)p, 2 * n);
+        return e == hipSuccess ? hipMemset(*p, 0, 2 * n) : e;
+    };
+    PIQMC_HIP(zeroed(&m->x, (size_t)B * lN));
+    PIQMC_HIP(zeroed(&m->h1, (size_t)B * l1));
+    PIQMC_HIP(zeroed(&m->h2, (size_t)B * l2));
     PIQMC_HIP(hipMalloc(&m->logits, 4 * (size_t)B * N));
-    PIQMC_HIP(hipMalloc(&m->dlog, 2 * (size_t)B * N));
-    PIQMC_HIP(hipMalloc(&m->dh2, 2 * (size_t)B * H2));
-    PIQMC_HIP(hipMalloc(&m->dh1, 2 * (size_t)B * H1));
-    PIQMC_HIP(hipMalloc(&m->tA, 2 * (size_t)B * Hm));
-    PIQMC_HIP(hipMalloc(&m->tB, 2 * (size_t)B * Hm));
+    PIQMC_HIP(zeroed(&m->dlog, (size_t)B * lN));
+    PIQMC_HIP(zeroed(&m->dh2, (size_t)B * l2));
+    PIQMC_HIP(zeroed(&m->dh1, (size_t)B * l1));
+    PIQMC_HIP(zeroed(&m->xt, (size_t)N * lB));
+    PIQMC_HIP(zeroed(&m->h1t, (size_t)H1 * lB));
+    PIQMC_HIP(zeroed(&m->h2t, (size_t)H2 * lB));
+    PIQMC_HIP(zeroed(&m->dlogt, (size_t)N * lB));
+    PIQMC_HIP(zeroed(&m->dh2t, (size_t)H2 * lB));
+    PIQMC_HIP(zeroed(&m->dh1t, (size_t)H1 * lB));
     PIQMC_HIP(hipMalloc(&m->nll, 8 * (size_t)B));
     PIQMC_HIP(hipMalloc(&m->s, (size_t)B * N));
+    // the zeroing runs on the null stream, the callers' streams need not wait for it
+    PIQMC_HIP(hipDeviceSynchronize());
     m->cap = B;
     return PIQMC_OK;
 }
 
 int grid1(size_t n) { return (int)std::min<size_t>((n + 255) / 256, 65535); }
 
-void transpose(const uint16_t *in, int R, int C, uint16_t *out, hipStream_t st)
+void transpose(const uint16_t *in, int R, int C, int ldi, uint16_t *out, int ldo, hipStream_t st)
 {
     dim3 g((C + 31) / 32, (R + 31) / 32), blk(32, 8);
-    transpose_bf16<<<g, blk, 0, st>>>(in, R, C, out);
+    transpose_bf16<<<g, blk, 0, st>>>(in, R, C, ldi, out, ldo);
 }
 
 // forward over m->x (bf16 spins) rows [0, B): h1, h2 (bf16), logits (fp32)
 void forward(piqmc_made *m, int B, hipStream_t st)
 {
-    gemm(m->x, m->N, m->wb[0], m->N, B, m->H1, m->N, m->b[0], 1, nullptr, m->h1, m->H1, st);
-    gemm(m->h1, m->H1, m->wb[1], m->H1, B, m->H2, m->H1, m->b[1], 1, nullptr, m->h2, m->H2, st);
-    gemm(m->h2, m->H2, m->wb[2], m->H2, B, m->N, m->H2, m->b[2], 0, m->logits, nullptr, m->N, st);
+    const int lN = up64(m->N), l1 = up64(m->H1), l2 = up64(m->H2);
+    gemm(m->x, lN, m->wb[0], lN, B, m->H1, m->N, m->b[0], 1, nullptr, m->h1, l1, st);
+    gemm(m->h1, l1, m->wb[1], l1, B, m->H2, m->H1, m->b[1], 1, nullptr, m->h2, l2, st);
+    gemm(m->h2, l2, m->wb[2], l2, B, m->N, m->H2, m->b[2], 0, m->logits, nullptr, m->N, st);
 }
 }  // namespace
 
@@ -709,16 +977,18 @@ extern "C" int piqmc_made_create(int N, int H1, int H2, uint64_t seed, piqmc_mad
         const double sc = 1.0 / sqrt((double)I);
         for (size_t t = 0; t < wv.size(); ++t) wv[t] = mk[t] ? (float)(uni() * sc) : 0.f;
         std::vector<float> zero_o(O, 0.f);
-        size_t nw = (size_t)O * I;
+        const size_t nw = (size_t)O * I, nwb = (size_t)O * up64(I), nwt = (size_t)I * up64(O);
         hipError_t e = hipSuccess;
         auto A = [&](void **p, size_t bytes) { if (e == hipSuccess) e = hipMalloc(p, bytes); };
         A((void **)&m->w[l], 4 * nw); A((void **)&m->mw[l], 4 * nw); A((void **)&m->vw[l], 4 * nw);
-        A((void **)&m->gw[l], 4 * nw); A((void **)&m->wb[l], 2 * nw); A((void **)&m->wt[l], 2 * nw);
+        A((void **)&m->gw[l], 4 * nw); A((void **)&m->wb[l], 2 * nwb); A((void **)&m->wt[l], 2 * nwt);
         A((void **)&m->mask[l], nw); A((void **)&m->b[l], 4 * O); A((void **)&m->mb[l], 4 * O);
         A((void **)&m->vb[l], 4 * O); A((void **)&m->gb[l], 4 * O);
         if (e == hipSuccess) e = hipMemcpy(m->w[l], wv.data(), 4 * nw, hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(m->mask[l], mk.data(), nw, hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemset(m->mw[l], 0, 4 * nw);
+        if (e == hipSuccess) e = hipMemset(m->wb[l], 0, 2 * nwb);
+        if (e == hipSuccess) e = hipMemset(m->wt[l], 0, 2 * nwt);
         if (e == hipSuccess) e = hipMemset(m->vw[l], 0, 4 * nw);
         if (e == hipSuccess) e = hipMemset(m->gw[l], 0, 4 * nw);
         if (e == hipSuccess) e = hipMemset(m->b[l], 0, 4 * O);
@@ -729,8 +999,8 @@ extern "C" int piqmc_made_create(int N, int H1, int H2, uint64_t seed, piqmc_mad
             return piqmc::hip_fail(e, "made_create");
         }
         // bf16 copies: an Adam step with zero gradient and zero lr refreshes them
-        adam_w<<<grid1(nw), 256>>>(m->w[l], m->mw[l], m->vw[l], m->gw[l], m->mask[l], O, I, 0.f, 0.9f, 0.999f,
-                                   1e-8f, 1.f, 1.f, m->wb[l], m->wt[l]);
+        adam_w<<<grid1(nw), 256>>>(m->w[l], m->mw[l], m->vw[l], m->gw[l], m->mask[l], O, I,
+                                   Adam{0.f, 0.9f, 0.999f, 1e-8f, 1.f, 1.f}, m->wb[l], up64(I), m->wt[l], up64(O));
     }
     PIQMC_HIP(hipDeviceSynchronize());
     *out = m;
@@ -746,8 +1016,8 @@ extern "C" int piqmc_made_destroy(piqmc_made *m)
         for (void *p : ps)
             if (p) (void)hipFree(p);
     }
-    void *bs[] = {m->x, m->h1, m->h2, m->logits, m->dlog, m->dh2, m->dh1, m->tA, m->tB, m->nll, m->s, m->rng,
-                  m->epoch_rows, m->nll_acc};
+    void *bs[] = {m->x, m->h1, m->h2, m->logits, m->dlog, m->dh2, m->dh1, m->xt, m->h1t, m->h2t, m->dlogt, m->dh2t,
+                  m->dh1t, m->nll, m->s, m->rng, m->epoch_nll};
     for (void *p : bs)
         if (p) (void)hipFree(p);
     if (m->gexec) (void)hipGraphExecDestroy(m->gexec);
@@ -794,9 +1064,9 @@ extern "C" int piqmc_made_logprob(piqmc_made *m, int B, const int8_t *s_dev, dou
     int rc = made_alloc_batch(m, B);
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
-    spins_to_bf16<<<grid1((size_t)B * m->N), 256, 0, st>>>(s_dev, (size_t)B * m->N, m->x);
+    spins_to_bf16<<<grid1((size_t)B * m->N), 256, 0, st>>>(s_dev, B, m->N, m->x, up64(m->N));
     forward(m, B, st);
-    output_nll<<<B, 256, 0, st>>>(m->logits, s_dev, B, m->N, 0.f, nullptr, m->nll, -1.0);
+    output_nll<<<B, 256, 0, st>>>(m->logits, s_dev, B, m->N, 0.f, nullptr, 0, m->nll, -1.0);
     PIQMC_HIP(hipMemcpyAsync(logq_dev, m->nll, 8 * (size_t)B, hipMemcpyDeviceToDevice, st));
     PIQMC_HIP(hipGetLastError());
     return PIQMC_OK;
@@ -805,77 +1075,147 @@ extern "C" int piqmc_made_logprob(piqmc_made *m, int B, const int8_t *s_dev, dou
 // Gradients of the mean NLL over B slices into the gradient buffers; returns
 // the mean NLL.  With lr > 0 also applies one Adam step.
 namespace {
-// One training step on the stream, no host synchronisation: the gradients
-// of the mean NLL of B slices, and an Adam step when lr > 0.  Per-row NLL in
-// m->nll.
-int train_core(piqmc_made *m, int B, const int8_t *s_dev, float lr, hipStream_t st)
+// K groups of the fused training product: those of the tile gemm() would take,
+// so that the order of summation is the same (a ragged K and the wide tiles
+// are summed in one group); -1 where 64 x 64 tiles are not what it would take
+// (the wide tiles win on large products).
+int train_groups(int M, int N, int K)
+{
+    const int tile = gemm_tile_choice(M, N, K);
+    if (K % PK == 0) return tile == 5 ? 4 : (tile == 4 ? 2 : (tile == 1 ? 1 : -1));
+    return (long long)((M + 63) / 64) * ((N + 63) / 64) <= 512 ? 1 : -1;
+}
+
+template <int NJ>
+void launch_train(const TrainJobs<NJ> &jobs, int kg, hipStream_t st)
+{
+    int grid = 0;
+    for (int i = 0; i < jobs.n; ++i) grid += jobs.blocks[i];
+    if (kg == 4) train_gemm<4, NJ><<<grid, 1024, 0, st>>>(jobs);
+    else if (kg == 2) train_gemm<2, NJ><<<grid, 512, 0, st>>>(jobs);
+    else train_gemm<1, NJ><<<grid, 256, 0, st>>>(jobs);
+}
+
+int tiles_of(int M, int N) { return ((M + GT - 1) / GT) * ((N + GT - 1) / GT); }
+
+// One training step on the stream, no host synchronisation: the gradients of
+// the mean NLL of the B slices s[perm[b0 + b]] (perm null: s[b0 + b]), and an
+// Adam step when lr > 0.  Per-row NLL in nll.
+int train_core(piqmc_made *m, int B, const int8_t *s, const int32_t *perm, int b0, float lr, double *nll,
+               hipStream_t st)
 {
     const int N = m->N, H1 = m->H1, H2 = m->H2;
-    spins_to_bf16<<<grid1((size_t)B * N), 256, 0, st>>>(s_dev, (size_t)B * N, m->x);
-    forward(m, B, st);
-    output_nll<<<B, 256, 0, st>>>(m->logits, s_dev, B, N, 1.f / (float)B, m->dlog, m->nll, 1.0);
-    // layer 3: dW2 = dlog^T h2, db2 = colsum(dlog), dh2 = dlog W2
-    transpose(m->dlog, B, N, m->tA, st);   // [N][B]
-    transpose(m->h2, B, H2, m->tB, st);    // [H2][B]
-    gemm(m->tA, B, m->tB, B, N, H2, B, nullptr, 0, m->gw[2], nullptr, H2, st);
-    col_sum_bf16<<<(N + 255) / 256, 256, 0, st>>>(m->dlog, B, N, m->gb[2]);
-    gemm(m->dlog, N, m->wt[2], N, B, H2, N, nullptr, 0, nullptr, m->dh2, H2, st);
-    relu_back<<<grid1((size_t)B * H2), 256, 0, st>>>(m->dh2, m->h2, (size_t)B * H2);
-    // layer 2
-    transpose(m->dh2, B, H2, m->tA, st);   // [H2][B]
-    transpose(m->h1, B, H1, m->tB, st);    // [H1][B]
-    gemm(m->tA, B, m->tB, B, H2, H1, B, nullptr, 0, m->gw[1], nullptr, H1, st);
-    col_sum_bf16<<<(H2 + 255) / 256, 256, 0, st>>>(m->dh2, B, H2, m->gb[1]);
-    gemm(m->dh2, H2, m->wt[1], H2, B, H1, H2, nullptr, 0, nullptr, m->dh1, H1, st);
-    relu_back<<<grid1((size_t)B * H1), 256, 0, st>>>(m->dh1, m->h1, (size_t)B * H1);
-    // layer 1
-    transpose(m->dh1, B, H1, m->tA, st);   // [H1][B]
-    transpose(m->x, B, N, m->tB, st);      // [N][B]
-    gemm(m->tA, B, m->tB, B, H1, N, B, nullptr, 0, m->gw[0], nullptr, N, st);
-    col_sum_bf16<<<(H1 + 255) / 256, 256, 0, st>>>(m->dh1, B, H1, m->gb[0]);
+    const int lN = up64(N), l1 = up64(H1), l2 = up64(H2), lB = up64(m->cap);
+    const int kf[3] = {train_groups(B, H1, N), train_groups(B, H2, H1), train_groups(B, N, H2)};
+    const int kd[2] = {train_groups(B, H1, H2), train_groups(B, H2, N)};  // dh1, dh2
+    const int kw[3] = {train_groups(H1, N, B), train_groups(H2, H1, B), train_groups(N, H2, B)};
+    bool fused = true;
+    for (int k : kf) fused = fused && k > 0;
+    for (int k : kd) fused = fused && k > 0;
+    for (int k : kw) fused = fused && k > 0;
+    Adam h = {lr, 0.9f, 0.999f, 1e-8f, 1.f, 1.f};
     if (lr > 0.f) {
         m->step++;
         m->ar_dirty = 1;
-        const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-        const float c1 = 1.f - powf(b1, (float)m->step), c2 = 1.f - powf(b2, (float)m->step);
-        for (int l = 0; l < 3; ++l) {
+        h.c1 = 1.f - powf(h.b1, (float)m->step);
+        h.c2 = 1.f - powf(h.b2, (float)m->step);
+    }
+    train_input<<<dim3((N + 63) / 64, (B + 63) / 64), 256, 0, st>>>(s, perm, b0, B, N, m->x, lN, m->xt, lB);
+    auto single = [&](TrainGemm g, int kg) {
+        TrainJobs<1> jobs = {};
+        g.K = up64(g.K);
+        jobs.j[0] = g;
+        jobs.n = 1;
+        jobs.blocks[0] = tiles_of(g.M, g.N);
+        launch_train(jobs, kg, st);
+    };
+    auto product = [&](const uint16_t *A, int lda, const uint16_t *W, int ldb, int cols, int K) {
+        TrainGemm g = {};
+        g.A = A; g.lda = lda; g.B = W; g.ldb = ldb; g.M = B; g.N = cols; g.K = K;
+        return g;
+    };
+    if (fused) {
+        TrainGemm g = product(m->x, lN, m->wb[0], lN, H1, N);
+        g.bias = m->b[0]; g.relu = 1; g.Cb = m->h1; g.ldc = l1; g.Ct = m->h1t; g.ldt = lB;
+        single(g, kf[0]);
+        g = product(m->h1, l1, m->wb[1], l1, H2, H1);
+        g.bias = m->b[1]; g.relu = 1; g.Cb = m->h2; g.ldc = l2; g.Ct = m->h2t; g.ldt = lB;
+        single(g, kf[1]);
+        g = product(m->h2, l2, m->wb[2], l2, N, H2);
+        g.bias = m->b[2]; g.Cf = m->logits; g.ldf = N;
+        single(g, kf[2]);
+    } else {
+        forward(m, B, st);
+    }
+    // whole tiles of the transposed gradients: rows past B are zeroed
+    train_nll<<<up64(B) / kNllRows, 256, 0, st>>>(m->logits, m->x, lN, B, N, 1.f / (float)B, m->dlog, lN, m->dlogt, lB, nll);
+    if (fused) {
+        TrainGemm g = product(m->dlog, lN, m->wt[2], lN, H2, N);
+        g.keep = m->h2; g.Cb = m->dh2; g.ldc = l2; g.Ct = m->dh2t; g.ldt = lB;
+        single(g, kd[1]);
+        g = product(m->dh2, l2, m->wt[1], l2, H1, H2);
+        g.keep = m->h1; g.ldc = l1; g.Ct = m->dh1t; g.ldt = lB;
+        single(g, kd[0]);
+    } else {
+        gemm(m->dlog, lN, m->wt[2], lN, B, H2, N, nullptr, 0, nullptr, m->dh2, l2, st);
+        relu_back<<<grid1((size_t)B * l2), 256, 0, st>>>(m->dh2, m->h2, (size_t)B * l2);
+        gemm(m->dh2, l2, m->wt[1], l2, B, H1, H2, nullptr, 0, nullptr, m->dh1, l1, st);
+        relu_back<<<grid1((size_t)B * l1), 256, 0, st>>>(m->dh1, m->h1, (size_t)B * l1);
+        transpose(m->h1, B, H1, l1, m->h1t, lB, st);
+        transpose(m->h2, B, H2, l2, m->h2t, lB, st);
+        transpose(m->dh2, B, H2, l2, m->dh2t, lB, st);
+        transpose(m->dh1, B, H1, l1, m->dh1t, lB, st);
+    }
+    const uint16_t *gt[3] = {m->dh1t, m->dh2t, m->dlogt}, *in[3] = {m->xt, m->h1t, m->h2t};
+    if (fused) {
+        for (int kg : {4, 2, 1}) {  // one launch per order of summation
+            TrainJobs<3> jobs = {};
+            jobs.h = h;
+            for (int l = 0; l < 3; ++l) {
+                if (kw[l] != kg) continue;
+                TrainGemm g = {};
+                g.A = gt[l]; g.lda = lB; g.B = in[l]; g.ldb = lB;
+                g.M = m->layers_out[l]; g.N = m->layers_in[l]; g.K = up64(B);
+                g.Cf = m->gw[l]; g.ldf = g.N;
+                g.step = lr > 0.f;
+                g.w = m->w[l]; g.m = m->mw[l]; g.v = m->vw[l]; g.mask = m->mask[l];
+                g.Cb = m->wb[l]; g.ldc = up64(g.N);
+                g.Ct = l ? m->wt[l] : nullptr; g.ldt = up64(g.M);  // the input layer's transpose is not used
+                g.gt = gt[l]; g.ldg = lB; g.units = g.M; g.rows = B; g.n64 = (g.M + 63) / 64;
+                g.gb = m->gb[l]; g.b = m->b[l]; g.bm = m->mb[l]; g.bv = m->vb[l];
+                jobs.blocks[jobs.n] = g.n64 + tiles_of(g.M, g.N);
+                jobs.j[jobs.n++] = g;
+            }
+            if (jobs.n) launch_train(jobs, kg, st);
+        }
+    } else {
+        for (int l = 2; l >= 0; --l) {
             const int O = m->layers_out[l], I = m->layers_in[l];
-            adam_w<<<grid1((size_t)O * I), 256, 0, st>>>(m->w[l], m->mw[l], m->vw[l], m->gw[l], m->mask[l], O, I, lr,
-                                                         b1, b2, eps, c1, c2, m->wb[l], m->wt[l]);
-            adam_b<<<(O + 255) / 256, 256, 0, st>>>(m->b[l], m->mb[l], m->vb[l], m->gb[l], O, lr, b1, b2, eps, c1, c2);
+            gemm(gt[l], lB, in[l], lB, O, I, B, nullptr, 0, m->gw[l], nullptr, I, st);
+            unit_sum_kernel<<<(O + 63) / 64, 256, 0, st>>>(gt[l], lB, O, B, m->gb[l]);
+        }
+        for (int l = 0; l < 3 && lr > 0.f; ++l) {
+            const int O = m->layers_out[l], I = m->layers_in[l];
+            adam_w<<<grid1((size_t)O * I), 256, 0, st>>>(m->w[l], m->mw[l], m->vw[l], m->gw[l], m->mask[l], O, I, h,
+                                                         m->wb[l], up64(I), m->wt[l], up64(O));
+            adam_b<<<(O + 255) / 256, 256, 0, st>>>(m->b[l], m->mb[l], m->vb[l], m->gb[l], O, h);
         }
     }
     PIQMC_HIP(hipGetLastError());
     return PIQMC_OK;
 }
 
-// rows data[perm[b0 + b]] -> out [B][N]
-__global__ void gather_rows(const int8_t *data, const int32_t *perm, int b0, int B, int N, int8_t *out)
+// sums[t] = sum of v[t n .. (t + 1) n), a workgroup each
+__global__ void __launch_bounds__(256) step_sums(const double *v, int n, double *sums)
 {
-    const size_t tot = (size_t)B * N;
-    for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < tot; t += (size_t)gridDim.x * blockDim.x) {
-        const int b = (int)(t / N), i = (int)(t % N);
-        out[t] = data[(size_t)perm[b0 + b] * N + i];
-    }
-}
-
-// acc[0] += sum of v[0..n) (one workgroup; launches on one stream run in order)
-__global__ void accumulate_sum(const double *v, int n, double *acc)
-{
-    __shared__ double red[16];
+    __shared__ double red[4];
     double t = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) t += v[i];
+    for (int i = threadIdx.x; i < n; i += 256) t += v[(size_t)blockIdx.x * n + i];
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int w = 0; w < (int)((blockDim.x + 63) >> 6); ++w) s += red[w];
-        acc[0] += s;
-    }
+    if (threadIdx.x == 0) sums[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
-
-__global__ void zero_double(double *p) { *p = 0.0; }
 }  // namespace
 
 extern "C" int piqmc_made_train_step(piqmc_made *m, int B, const int8_t *s_dev, float lr, double *mean_nll,
@@ -885,7 +1225,7 @@ extern "C" int piqmc_made_train_step(piqmc_made *m, int B, const int8_t *s_dev, 
     int rc = made_alloc_batch(m, B);
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
-    rc = train_core(m, B, s_dev, lr, st);
+    rc = train_core(m, B, s_dev, nullptr, 0, lr, m->nll, st);
     if (rc) return rc;
     if (mean_nll) {
         std::vector<double> h(B);
@@ -906,33 +1246,33 @@ extern "C" int piqmc_made_train_epoch(piqmc_made *m, int n, const int8_t *data_d
 {
     if (!m || n < 1 || batch < 1 || batch > n || !data_dev || !perm_dev)
         return piqmc::set_error(PIQMC_EINVAL, "made_train_epoch: bad args");
-    // the batch rows live past the sampler's rows in a buffer of its own
     int rc = made_alloc_batch(m, batch);
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
-    if (!m->epoch_rows || m->epoch_cap < batch) {
-        if (m->epoch_rows) PIQMC_HIP(hipFree(m->epoch_rows));
-        m->epoch_rows = nullptr;
-        m->epoch_cap = 0;
-        PIQMC_HIP(hipMalloc(&m->epoch_rows, (size_t)batch * m->N));
-        m->epoch_cap = batch;
-    }
-    if (!m->nll_acc) PIQMC_HIP(hipMalloc(&m->nll_acc, sizeof(double)));
-    zero_double<<<1, 1, 0, st>>>(m->nll_acc);
     const int steps = n / batch;
-    for (int t = 0; t < steps; ++t) {
-        gather_rows<<<grid1((size_t)batch * m->N), 256, 0, st>>>(data_dev, perm_dev, t * batch, batch, m->N,
-                                                                 m->epoch_rows);
-        rc = train_core(m, batch, m->epoch_rows, lr, st);
-        if (rc) return rc;
-        accumulate_sum<<<1, 256, 0, st>>>(m->nll, batch, m->nll_acc);
+    // per-row NLL of every step, then the steps' sums
+    const size_t need = (size_t)steps * batch + steps;
+    if (m->epoch_cap < need) {
+        if (m->epoch_nll) PIQMC_HIP(hipFree(m->epoch_nll));
+        m->epoch_nll = nullptr;
+        m->epoch_cap = 0;
+        PIQMC_HIP(hipMalloc(&m->epoch_nll, sizeof(double) * need));
+        m->epoch_cap = need;
     }
+    double *sums = m->epoch_nll + (size_t)steps * batch;
+    for (int t = 0; t < steps; ++t) {
+        rc = train_core(m, batch, data_dev, perm_dev, t * batch, lr, m->epoch_nll + (size_t)t * batch, st);
+        if (rc) return rc;
+    }
+    step_sums<<<steps, 256, 0, st>>>(m->epoch_nll, batch, sums);
     PIQMC_HIP(hipGetLastError());
     if (mean_nll) {
-        double h = 0.0;
-        PIQMC_HIP(hipMemcpyAsync(&h, m->nll_acc, sizeof(double), hipMemcpyDeviceToHost, st));
+        std::vector<double> h(steps);
+        PIQMC_HIP(hipMemcpyAsync(h.data(), sums, sizeof(double) * steps, hipMemcpyDeviceToHost, st));
         PIQMC_HIP(hipStreamSynchronize(st));
-        *mean_nll = h / ((double)steps * batch);
+        double t = 0.0;
+        for (double v : h) t += v;
+        *mean_nll = t / ((double)steps * batch);
     }
     return PIQMC_OK;
 }
@@ -957,13 +1297,13 @@ extern "C" int piqmc_made_sample(piqmc_made *m, int B, uint64_t seed, uint32_t r
     // graph and replayed.
     auto chain = [&](hipStream_t s) {
         fill_i8<<<grid1((size_t)B * N), 256, 0, s>>>(m->s, (size_t)B * N, 1);  // placeholders beyond the prefix
-        spins_to_bf16<<<grid1((size_t)B * N), 256, 0, s>>>(m->s, (size_t)B * N, m->x);
+        spins_to_bf16<<<grid1((size_t)B * N), 256, 0, s>>>(m->s, B, N, m->x, up64(N));
         for (int d = 0; d < N; ++d) {
             forward(m, B, s);
-            sample_step<<<(B + 255) / 256, 256, 0, s>>>(m->logits, B, N, d, m->rng, m->s, m->x);
+            sample_step<<<(B + 255) / 256, 256, 0, s>>>(m->logits, B, N, d, m->rng, m->s, m->x, up64(N));
         }
         forward(m, B, s);
-        output_nll<<<B, 256, 0, s>>>(m->logits, m->s, B, N, 0.f, nullptr, m->nll, -1.0);
+        output_nll<<<B, 256, 0, s>>>(m->logits, m->s, B, N, 0.f, nullptr, 0, m->nll, -1.0);
     };
     if (m->use_graph) {
         if (!m->gs) {

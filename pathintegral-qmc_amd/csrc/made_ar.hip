@@ -91,17 +91,17 @@ __global__ void ar_tables_kernel(int N, int H1, int H2, int DS, int JM, const ui
         if (t < n0) {
             const int s = (int)(t % ZSP), ln = (int)((t / ZSP) % 64), e = (int)(t / ((size_t)64 * ZSP));
             const int k = s < ZS ? ar_unit((s % DS) * 64 + ln, s / DS, N, H1) : -1;
-            w0t[t] = k >= 0 ? wb0[(size_t)k * N + e] : (uint16_t)0;
+            w0t[t] = k >= 0 ? wb0[(size_t)k * ((N + 63) & ~63) + e] : (uint16_t)0;
         } else if (t < n0 + n1) {
             const size_t u = t - n0;
             const int s = (int)(u % ZSP), ln = (int)((u / ZSP) % 64), k1 = (int)(u / ((size_t)64 * ZSP));
             const int k2 = s < ZS ? ar_unit((s % DS) * 64 + ln, s / DS, N, H2) : -1;
-            w1t[u] = k2 >= 0 ? wb1[(size_t)k2 * H1 + k1] : (uint16_t)0;
+            w1t[u] = k2 >= 0 ? wb1[(size_t)k2 * ((H1 + 63) & ~63) + k1] : (uint16_t)0;
         } else if (t < n0 + n1 + n2) {
             const size_t u = t - n0 - n1;
             const int q = (int)(u % DSP), ln = (int)((u / DSP) % 64), k2 = (int)(u / ((size_t)64 * DSP));
             const int d = q * 64 + ln;  // logit d + 1
-            w2t[u] = (q < DS && d <= N - 2) ? wb2[(size_t)(d + 1) * H2 + k2] : (uint16_t)0;
+            w2t[u] = (q < DS && d <= N - 2) ? wb2[(size_t)(d + 1) * ((H2 + 63) & ~63) + k2] : (uint16_t)0;
         } else {
             const size_t u = t - n0 - n1 - n2;
             const int ln = (int)(u / (2 * ZS + DS)), c = (int)(u % (2 * ZS + DS));

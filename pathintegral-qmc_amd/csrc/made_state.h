@@ -9,14 +9,15 @@ struct piqmc_made {
     int N = 0, H1 = 0, H2 = 0, cap = 0;  // cap = max batch rows of the buffers
     int layers_in[3], layers_out[3];
     float *w[3] = {}, *b[3] = {}, *mw[3] = {}, *vw[3] = {}, *mb[3] = {}, *vb[3] = {};
-    uint16_t *wb[3] = {}, *wt[3] = {};
+    uint16_t *wb[3] = {}, *wt[3] = {};   // bf16 [out][in], [in][out], row pitches rounded up to 64, zeros past the sizes
     uint8_t *mask[3] = {};
     float *gw[3] = {}, *gb[3] = {};
-    // activations [cap][*]
+    // activations [cap][*], row pitches (but the logits') rounded up to 64, zeros past the sizes
     uint16_t *x = nullptr, *h1 = nullptr, *h2 = nullptr;
     float *logits = nullptr;
     uint16_t *dlog = nullptr, *dh2 = nullptr, *dh1 = nullptr;
-    uint16_t *tA = nullptr, *tB = nullptr;  // transposes for weight gradients
+    // transposes for the weight gradients [units][cap rounded up to 64]
+    uint16_t *xt = nullptr, *h1t = nullptr, *h2t = nullptr, *dlogt = nullptr, *dh2t = nullptr, *dh1t = nullptr;
     double *nll = nullptr;
     int8_t *s = nullptr;
     int step = 0;
@@ -27,10 +28,9 @@ struct piqmc_made {
     hipGraphExec_t gexec = nullptr;
     int gB = 0;
     int use_graph = 1;
-    // epoch training: the gathered batch rows and the running NLL sum
-    int8_t *epoch_rows = nullptr;
-    int epoch_cap = 0;
-    double *nll_acc = nullptr;
+    // epoch training: every row's NLL, then every step's sum
+    double *epoch_nll = nullptr;
+    size_t epoch_cap = 0;
     // fused autoregressive sampler: the weights in its lane layout, rebuilt
     // from the bf16 weights whenever they change (ar_dirty)
     int ar_dirty = 1;
