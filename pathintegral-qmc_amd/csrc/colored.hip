@@ -30,6 +30,7 @@
 #include <string>
 #include <type_traits>
 
+#include "dense_block.h"
 #include "piqmc_internal.h"
 #include "sparse.h"
 
@@ -2555,7 +2556,11 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         int pw = 4;
         size_t lwg = 0;
         bool fields_auto = false;
-        if (pb->dense_variant == 0) {
+        const bool block_sweep = (pb->dense_variant == 0 || pb->dense_variant == 6) && piqmc::block_applies(pb);
+        if (block_sweep) {
+            // blocks of spins, both parities at once (dense_block.hip): faster at
+            // every slice and replica count measured (2 to 8192 replicas)
+        } else if (pb->dense_variant == 0) {
             // cached fields while replicas are few (256-spin SK, P=128: 33 ms
             // against 46 ms pipelined at 4 replicas, 20 against 18 at 64)
             fields_auto = pb->exact_rows && pb->fields_ok && pb->Z <= kFieldsMaxRow && R <= 32 &&
@@ -2588,8 +2593,8 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
                                                       "summable rows and a row that fits the LDS");
             wg = true;
         }
-        const bool fields = pb->dense_variant == 6 || fields_auto;
-        if (!wg && !fields && lds > 160 * 1024) return piqmc::set_error(PIQMC_EINVAL, "dense sweep: state exceeds LDS");
+        const bool fields = !block_sweep && (pb->dense_variant == 6 || fields_auto);
+        if (!wg && !fields && !block_sweep && lds > 160 * 1024) return piqmc::set_error(PIQMC_EINVAL, "dense sweep: state exceeds LDS");
         float *d_jp = nullptr;  // [S] J_perp, then [S] temperatures
         WT *d_packed = nullptr;
         double *d_fields = nullptr;
@@ -2608,7 +2613,13 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         a.jperp = d_jp; a.rows = pb->d_rows; a.order = pb->d_order; a.prevj = pb->d_prevj;
         a.packed = d_packed; a.etrace = etrace; a.fields = d_fields;
         piqmc::timing_begin(st);
-        if (fields) {
+        if (block_sweep) {
+            piqmc::BlockArgs b = piqmc::block_args(pb);
+            b.P = P; b.W = W; b.S = S; b.M = M; b.R = R;
+            b.key0 = a.key0; b.key1 = a.key1; b.replica_base = rbase; b.sweep_base = sbase;
+            b.jperp = d_jp; b.temps = d_jp + S; b.packed = d_packed; b.etrace = etrace;
+            if ((rc = piqmc::block_launch(b, st))) return rc;
+        } else if (fields) {
             // one replica per wavefront, as many per workgroup as block and LDS allow
             const size_t per = dense_fields_bytes(N, W, sizeof(WT));
             const int wf = std::max(1, std::min(std::min(wpb, 4), (int)((160 * 1024) / per)));

@@ -14,6 +14,7 @@
 
 #include <tuple>
 #include <cstring>
+#include "dense_block.h"
 #include "piqmc_internal.h"
 #include "sparse.h"
 
@@ -275,6 +276,7 @@ static int upload_coloring(piqmc_problem &p)
     }
     PIQMC_HIP(hipMalloc(&p.d_prevj, sizeof(double) * N));
     PIQMC_HIP(hipMemcpy(p.d_prevj, prevj.data(), sizeof(double) * N, hipMemcpyHostToDevice));
+    if (const int rc = piqmc::block_upload(p, order)) return rc;
     if (!p.pmj && !p.pmjf) {
         const int rc = piqmc::sparse_upload(p, order);
         if (rc) return rc;
@@ -490,6 +492,7 @@ extern "C" int piqmc_problem_destroy(piqmc_problem *p)
 {
     if (!p) return PIQMC_OK;
     piqmc::sparse_free(*p);
+    if (p->d_block) (void)hipFree(p->d_block);
     if (p->d_rows) (void)hipFree(p->d_rows);
     if (p->d_jd) (void)hipFree(p->d_jd);
     if (p->d_order) (void)hipFree(p->d_order);

@@ -88,6 +88,9 @@ struct piqmc_problem {
     // the problem has no such tables).
     piqmc::SparseTab sparse;
     int sparse_rows = 0;
+    // The blocked dense sweep's tables (null: it does not apply).
+    unsigned char *d_block = nullptr;
+    float block_bound = 0.0f;
     unsigned char *d_sparse = nullptr;  // what the tables' arrays are parts of
 };
 

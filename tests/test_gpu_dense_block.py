@@ -1,0 +1,63 @@
+"""The blocked dense sweep, bit for bit against the CPU twin: partial blocks,
+one block only, every register width, both word sizes, fields, traces and the
+schedules on which its float thresholds do not apply."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _dense(N, rng, sparse=False, field=False):
+    """Couplings on a grid of 2^-12 (every row sums exactly), some zero."""
+    from piqmc import instances
+    r, c = np.triu_indices(N, 1)
+    v = np.round(rng.randn(r.size) / np.sqrt(N) * 4096) / 4096
+    if sparse:
+        v[rng.rand(v.size) < 0.5] = 0.0
+    if field:
+        r, c = np.r_[r, np.arange(N)], np.r_[c, np.arange(N)]
+        v = np.r_[v, np.round(rng.randn(N) * 1024) / 4096]
+    return instances.neighbors(N, r, c, v)
+
+
+@pytest.mark.parametrize("N", [5, 16, 17, 33, 64, 100, 130, 200, 256])
+@pytest.mark.parametrize("P,T,M", [(2, 0.2, 1), (18, 1 / 18, 2), (64, 1 / 64, 1), (66, 0.5, 1), (128, 1 / 128, 1)])
+def test_blocked_sweep_matches_oracle(gpu, N, P, T, M):
+    import torch
+    from piqmc import device
+    rng = np.random.RandomState(N * 131 + P)
+    nbs = _dense(N, rng, sparse=N == 33, field=N in (17, 100))
+    pb = device.Problem(nbs)
+    pb.set_sweep_path("dense")
+    assert pb.exact_rows
+    R, color = 2, pb.coloring()
+    # the last field has infinite J_perp: every decision is made in double
+    sched = np.r_[np.linspace(3.0, 1e-8, 5), 0.0]
+    init = (2 * rng.randint(2, size=(R, P, N)) - 1).astype(np.int8)
+    for trace in (False, True):
+        d = torch.from_numpy(init.copy()).to(gpu)
+        et = pb.qa_colored(d, sched, M, T, 7 + P, replica_base=3, sweep_base=9, trace=trace)
+        for r in range(R):
+            ref = init[r].copy()
+            etr = O.qa_colored(sched, M, P, T, ref, nbs, color, pb.ncolors, 7 + P, replica=3 + r, sweep_base=9,
+                               trace=True)
+            assert np.array_equal(d[r].cpu().numpy(), ref)
+            if trace:
+                np.testing.assert_allclose(et[r].cpu().numpy(), etr, rtol=1e-12, atol=1e-9)
+
+
+@pytest.mark.parametrize("N,C", [(24, 10), (70, 128)])
+def test_blocked_chains_match_oracle(gpu, N, C):
+    import torch
+    from piqmc import device
+    rng = np.random.RandomState(N)
+    nbs = _dense(N, rng)
+    pb = device.Problem(nbs)
+    sched = np.linspace(2.0, 0.05, 6)
+    ref = (2 * rng.randint(2, size=(C, N)) - 1).astype(np.int8)
+    d = torch.from_numpy(ref.copy()).to(gpu)
+    pb.sa_colored(d, sched, 2, seed=5)
+    O.sa_colored(sched, 2, ref, nbs, pb.coloring(), pb.ncolors, 5)
+    assert np.array_equal(d.cpu().numpy(), ref)
