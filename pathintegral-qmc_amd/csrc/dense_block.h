@@ -27,6 +27,11 @@ struct BlockArgs {
 inline bool block_applies(const piqmc_problem *p) { return p->d_block != nullptr; }
 BlockArgs block_args(const piqmc_problem *p);  // N and the problem's tables filled in
 int block_launch(const BlockArgs &a, hipStream_t st);
+// Batches: LDS of a job's replica, and the persistent launch over items (job,
+// replica) on device arrays.
+size_t block_item_lds(const BlockArgs &a);
+int block_batch_prepare(size_t lds);
+void block_batch_launch(const BlockArgs *jobs, const int2 *items, int n, int *head, int grid, size_t lds, hipStream_t st);
 int block_upload(piqmc_problem &p, const std::vector<int32_t> &order);
 
 }  // namespace piqmc

@@ -264,8 +264,9 @@ __device__ void block_sweep(const BlockArgs &a, int r, unsigned char *smem)
         }
         wave_sync();
         const int l = lane & 31;
+        constexpr int kPasses = sizeof(WT) == 4 ? 4 : 2;  // (64-bit words: the fields leave few registers)
         const float cT = fin ? -0.34657359027997264f * T : __uint_as_float(0x7fc00000u);  // NaN: decided in double
-#pragma unroll
+#pragma unroll kPasses
         for (int v = 0; v < 4; ++v) {
             const uint32_t u = __brev(transpose32(sc[v * 64 + lane], l));
             const int pos = sizeof(WT) == 4 ? 2 * v + (lane >> 5) : v, m = sizeof(WT) == 4 ? l : lane;
@@ -279,15 +280,7 @@ __device__ void block_sweep(const BlockArgs &a, int r, unsigned char *smem)
     // The team's place: block c of sweep (step s, m of it), the index of which
     // in the call is x; `buf` holds its thresholds and block couplings.
     const int total = a.S * a.M * nbk;
-    // rows on their way to LDS: the helpers' 16-byte groups of the coming block
-    constexpr int nth = (kTeam - 1) * 64, kV = 64 * KS / 4, kG = (kB * kV + nth - 1) / nth;
-    const int t0 = (tw - 1) * 64 + lane;
-    f4 rv[kG];
-    if (tw > 0) {
-#pragma unroll
-        for (int y = 0; y < kG; ++y)
-            rv[y] = reinterpret_cast<const f4 *>(a.j2)[min(t0 + y * nth, min(kB, N) * kV - 1)];
-    }
+    constexpr int kV = 64 * KS / 4;  // 16-byte groups per row
     int x = 0, c = 0, m = 0, s = 0, buf = 0;
     float T = total > 0 ? a.temps[0] : 0.0f, jp = total > 0 ? a.jperp[0] : 0.0f;
     if (total > 0) {
@@ -435,21 +428,20 @@ __device__ void block_sweep(const BlockArgs &a, int r, unsigned char *smem)
                 __builtin_amdgcn_s_setprio(0);
             } else if (on) {
                 // this block's rows for the updates, the next block's couplings and draws
-                f4 *dst = reinterpret_cast<f4 *>(rows);
-                const int last = max(nq * kV - 1, 0);  // past it a lane repeats the last group
-#pragma unroll
-                for (int y = 0; y < kG; ++y) dst[min(t0 + y * nth, last)] = rv[y];
-                if (more) {  // the next block's, a step ahead of their use
-                    const f4 *nx = reinterpret_cast<const f4 *>(a.j2 + (size_t)cn * kB * 64 * KS);
-                    const int ln = max(min(kB, N - cn * kB) * kV - 1, 0);
-#pragma unroll
-                    for (int y = 0; y < kG; ++y) rv[y] = nx[min(t0 + y * nth, ln)];
-                }
+                // (straight to LDS, a wavefront's 64 groups at a time; groups past
+                // the block's rows repeat its last one)
+                const f4 *src = reinterpret_cast<const f4 *>(a.j2 + (size_t)c * kB * 64 * KS);
+                const int last = nq * kV - 1;  // (below 0 in the empty block of a single one)
+                for (int y = tw - 1; y < kB * kV / 64 && last >= 0; y += kTeam - 1)
+                    __builtin_amdgcn_global_load_lds(
+                        (const __attribute__((address_space(1))) void *)(src + min(y * 64 + lane, last)),
+                        (__attribute__((address_space(3))) void *)(rows + y * 256), 16, 0, 0);
                 if (more) {
                     if (tw == 1) stage_jb(cn, buf ^ 1);
                     for (int task = kTeam - 1 - tw; task < kTasks; task += kTeam - 1)
                         draw(task, cn, a.sweep_base + (uint32_t)(sn * a.M + mn), Tn, finite(Tn, jpn), buf ^ 1);
                 }
+                __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the rows are in LDS before the barrier
             }
             __syncthreads();
             if (on) {
@@ -530,6 +522,36 @@ __global__ void __launch_bounds__(128 * kTeam) block_kernel(BlockArgs a)
     block_sweep<WT, KS>(a, blockIdx.x, smem);
 }
 
+// Replicas of a batch's jobs from a device counter, longest first: resident
+// workgroups leave once the counter has passed the items.
+template <typename WT>
+__device__ void block_item(const BlockArgs &a, int r, unsigned char *smem)
+{
+    switch ((a.N + 63) / 64) {
+    case 1: block_sweep<WT, 1>(a, r, smem); break;
+    case 2: block_sweep<WT, 2>(a, r, smem); break;
+    case 3: block_sweep<WT, 3>(a, r, smem); break;
+    default: block_sweep<WT, 4>(a, r, smem); break;
+    }
+}
+__global__ void __launch_bounds__(128 * kTeam) batch_block_kernel(const BlockArgs *jobs, const int2 *items, int n, int *head)
+{
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int cur;
+    for (;;) {
+        __syncthreads();
+        if (threadIdx.x == 0) cur = atomicAdd(head, 1);
+        __syncthreads();
+        const int it = __builtin_amdgcn_readfirstlane(cur);
+        if (it >= n) break;
+        const int2 item = items[it];
+        const BlockArgs &a = jobs[__builtin_amdgcn_readfirstlane(item.x)];
+        const int r = __builtin_amdgcn_readfirstlane(item.y);
+        if (a.W <= 32) block_item<uint32_t>(a, r, smem);
+        else block_item<uint64_t>(a, r, smem);
+    }
+}
+
 template <typename WT, int KS>
 int launch(const BlockArgs &a, hipStream_t st)
 {
@@ -571,6 +593,19 @@ BlockArgs block_args(const piqmc_problem *p)
 int block_launch(const BlockArgs &a, hipStream_t st)
 {
     return a.W <= 32 ? launch_slots<uint32_t>(a, st) : launch_slots<uint64_t>(a, st);
+}
+
+size_t block_item_lds(const BlockArgs &a) { return block_lds(a.N, a.W <= 32 ? 4 : 8); }
+
+int block_batch_prepare(size_t lds)
+{
+    PIQMC_HIP(hipFuncSetAttribute((const void *)batch_block_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    return PIQMC_OK;
+}
+
+void block_batch_launch(const BlockArgs *jobs, const int2 *items, int n, int *head, int grid, size_t lds, hipStream_t st)
+{
+    batch_block_kernel<<<grid, 128 * kTeam, lds, st>>>(jobs, items, n, head);
 }
 
 // [diag | twice the couplings | those within blocks] by color position, where the blocked sweep
