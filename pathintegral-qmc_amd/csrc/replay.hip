@@ -3,8 +3,11 @@
 //
 // A replica's sweep is a strictly sequential Markov chain (the reference keeps
 // a running ediff across the spins of a slice, D2, and draws libc rand() only
-// on the rejection branch), so one lane owns one replica and the replicas of
-// a wave advance in lockstep.  A few lanes per wave own replicas (a chain's
+// on the rejection branch).  replay_wave_kernel gives a replica a wavefront, whose
+// lanes work ahead of the chain; it takes the calls whose replicas do not fill the
+// chip's lanes.  replay_kernel takes the others and the dense problems: one lane
+// owns one replica and the replicas of a wave advance in lockstep.  A few lanes
+// per wave own replicas (a chain's
 // speed is its latency, so replicas are spread over every SIMD) and the waves
 // of a workgroup share one LDS copy of the neighbour rows.  Per replica the
 // kernel keeps, bit-packed in LDS with slot-interleaved words (conflict-free):
@@ -70,6 +73,13 @@ __host__ __device__ inline size_t replay_words(int nreg, int Wn, int Ls)
 {
     const size_t rs = (size_t)replay_region_words(Wn, Ls);
     return (rs + nreg * rs + (size_t)31 * Ls + 1) & ~(size_t)1;
+}
+
+// LDS words of a wavefront of replay_wave_kernel: the swept slice, slices 1 and
+// P - 1, the sweep's permutation.
+__host__ __device__ inline size_t replay_wave_words(int N, int Wn, bool sa)
+{
+    return (size_t)(sa ? 1 : 3) * Wn + (size_t)(N + 1) / 2;
 }
 
 // LDS byte address of a pointer into shared memory, and a word read at one.
@@ -332,6 +342,275 @@ __global__ void replay_kernel(ReplayArgs a)
     a.ties[r] = nt;
 }
 
+// One replica per wavefront.  What bounds a call is one replica's chain of
+// attempts: with a lane to itself a replica spends about 730 cycles on one, LDS
+// round trips for the spins, the terms' arithmetic, the exponential, a division.
+// Here the lanes of its wavefront share that work out over the next 64 attempts:
+//   - Lane a reads attempt a's row and spins and forms its terms, all but the
+//     running sum.  The chain is then the sum in the reference's order, handed
+//     from lane to lane, and a flip changes the sign of the terms in which later
+//     lanes named that spin.
+//   - The rand() stream does not depend on the state, only how much of it is used
+//     does: a block of 31 outputs (the ring's length) is a prefix sum over lanes,
+//     v[n] = v[n - 31] + v[n - 3], and each lane turns its output into the
+//     threshold T ln(u) on the running sum, in float.  Only a sum within the
+//     float's error of the threshold computes the exponential and compares in
+//     double (and counts near ties, which all lie there).
+//   - Because the sum runs on over a slice, attempts are rejected in long runs (70
+//     to 220 at a time) and flip without a draw in runs.  So the sums of up to 31
+//     attempts are formed as if all were rejected, and one comparison finds the
+//     first that may not be; flips without a draw follow each other attempt by
+//     attempt.
+// A rejected attempt costs its dependent additions, about 50 cycles; 96 in all at
+// 64 spins.  Kernel time, a lane each and a wavefront each: 64-spin lattice, P=20,
+// one replica, 100 sweeps, 36.0 and 5.1 ms; 1024 spins, P=64, 2048 replicas, 5
+// sweeps, 103.6 and 22.0 ms; 3600 spins, P=8, one replica, 20 sweeps, 486 and 21 ms.
+template <bool SA, int ZK>
+__global__ void __launch_bounds__(256) replay_wave_kernel(ReplayArgs a)
+{
+    extern __shared__ uint32_t sm[];
+    const int N = a.N, P = a.P, Z = a.Z, Wn = a.Wn, R = a.R, lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = blockIdx.x * (blockDim.x >> 6) + wv;
+    if (r >= R) return;  // no barriers: a wavefront uses its own part of the LDS
+    uint32_t *cur = sm + (size_t)wv * replay_wave_words(N, Wn, SA), *s1 = cur + Wn, *sp = s1 + Wn;
+    uint16_t *perm = reinterpret_cast<uint16_t *>(SA ? s1 : sp + Wn);
+    if constexpr (SA) s1 = sp = cur;
+    else if (P == 2) sp = s1;
+    auto sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    auto load = [&](uint32_t *reg, int k) {
+        for (int w = lane; w < Wn; w += 64) reg[w] = a.bits[((size_t)k * Wn + w) * R + r];
+    };
+    auto store = [&](const uint32_t *reg, int k) {
+        for (int w = lane; w < Wn; w += 64) a.bits[((size_t)k * Wn + w) * R + r] = reg[w];
+    };
+    if constexpr (SA) {
+        load(cur, 0);
+    } else {
+        load(s1, 1);
+        if (P != 2) load(sp, P - 1);
+    }
+    // rand(): output n of the current block of 31 (ring position f0 + n) is held by
+    // lane 16 (n % 3) + n / 3: a row of the wavefront is a chain of the recurrence.
+    // `rv` is the block, `ro` the one before; nu of the block's outputs are used.
+    const uint32_t f0 = a.rstate[(size_t)r * 32 + 31] % 31u;
+    const int on = 3 * (lane & 15) + (lane >> 4);
+    const bool out = lane < 48 && on < 31;
+    const int slot = (int)((f0 + (uint32_t)(out ? on : 0)) % 31u);
+    uint32_t rv = out ? a.rstate[(size_t)r * 32 + slot] : 0u, ro = rv;
+    // and in order: lane n has output n, and its thresholds on the running sum
+    const int lin = 4 * (16 * (min(lane, 30) % 3) + min(lane, 30) / 3);
+    uint32_t rl = 0;
+    float T = SA ? 0.0f : a.temp, hi = 0.0f, lo = 0.0f;
+    int nu = 0;
+    unsigned long long nd = 0;
+    uint32_t nt = 0;
+    auto thresholds = [&] {
+        const uint32_t x = rl >> 1;
+        // ln(u) to 1e-6 of a value of at most 21.5, and the quotient e / T rounds to
+        // 1.3e-6: 3e-5 T is wide.  u = 0 and a temperature that is not finite and
+        // positive leave every sum to the comparison in double.
+        const float L = T * 0.69314718f * __builtin_amdgcn_logf((float)x * 4.656612873077393e-10f), g = 3e-5f * T;
+        const bool fin = T > 0.0f && T < INFINITY && x != 0u;
+        hi = fin ? L + g : INFINITY;
+        lo = fin ? L - g : -INFINITY;
+    };
+    auto next_block = [&] {
+        ro = rv;
+        // v[n] = old[n] + v[n - 3]: a prefix sum along each row, begun by the last
+        // three outputs of the block before (28, 29 and 30)
+        const uint32_t l28 = (uint32_t)__builtin_amdgcn_readlane((int)rv, 25);
+        const uint32_t l29 = (uint32_t)__builtin_amdgcn_readlane((int)rv, 41);
+        const uint32_t l30 = (uint32_t)__builtin_amdgcn_readlane((int)rv, 10);
+        uint32_t x = rv + (lane == 0 ? l28 : lane == 16 ? l29 : lane == 32 ? l30 : 0u);
+        x += (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x111, 0xf, 0xf, true);  // row_shr 1, 2, 4, 8
+        x += (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x112, 0xf, 0xf, true);
+        x += (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x114, 0xf, 0xf, true);
+        x += (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x118, 0xf, 0xf, true);
+        rv = out ? x : 0u;
+        rl = (uint32_t)__builtin_amdgcn_ds_bpermute(lin, (int)rv);
+        nu = 0;
+        thresholds();
+    };
+    // lane l - 1's value, 0 in lane 0
+    auto lane_before = [](float x) __attribute__((always_inline)) {
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x138, 0xf, 0xf, true));  // wave_shr 1
+    };
+    next_block();
+    const int nslice = SA ? 1 : P;
+    const int nb64 = (N + 63) / 64;
+    for (int s = 0; s < a.S; ++s) {
+        const float sv = a.steps[s];
+        const uint32_t svm2 = __float_as_uint(-2.0f * sv);  // exact
+        if constexpr (SA) {
+            T = sv;
+            thresholds();
+        }
+        for (int m = 0; m < a.M; ++m) {
+            const uint16_t *pg = a.perms + (size_t)(s * a.M + m) * N * R + r;
+            sync();
+            for (int t0 = 0; t0 < N; t0 += 256) {  // four loads in flight a lane
+                uint16_t v[4];
+#pragma unroll
+                for (int y = 0; y < 4; ++y) v[y] = pg[(size_t)min(t0 + 64 * y + lane, N - 1) * R];
+#pragma unroll
+                for (int y = 0; y < 4; ++y)
+                    if (t0 + 64 * y + lane < N) perm[t0 + 64 * y + lane] = v[y];
+            }
+            sync();
+            // the next 64 attempts' rows, and the next slice's first 64 words, are
+            // read a batch and a slice ahead
+            int in = (int)perm[min(lane, N - 1)];
+            int2 rn[ZK];
+#pragma unroll
+            for (int z = 0; z < ZK; ++z) rn[z] = a.rows[(size_t)in * Z + min(z, Z - 1)];
+            const int w0 = min(lane, Wn - 1);
+            uint32_t ahead = a.bits[(size_t)w0 * R + r];
+            for (int k = 0; k < nslice; ++k) {
+                uint32_t *reg = SA ? cur : (k == 1 ? s1 : (k == P - 1 ? sp : cur));
+                const bool own = !SA && reg == cur;
+                if (own) {
+                    if (lane < Wn) cur[lane] = ahead;
+                    for (int w = 64 + lane; w < Wn; w += 64) cur[w] = a.bits[((size_t)k * Wn + w) * R + r];
+                }
+                sync();
+                ahead = a.bits[((size_t)min(k + 1, nslice - 1) * Wn + w0) * R + r];
+                float base = 0.0f;  // the running sum after the batches before
+                for (int b = 0; b < nb64; ++b) {
+                    const int i = in;
+                    int nb[ZK];
+                    uint32_t t[ZK];
+                    const uint32_t xi = (reg[i >> 5] >> (i & 31)) << 31;
+#pragma unroll
+                    for (int z = 0; z < ZK; ++z) {
+                        const int j = rn[z].x;
+                        const bool real = z < Z;
+                        const uint32_t xj = j == i ? 0u : (reg[j >> 5] >> (j & 31)) << 31;
+                        // -2 s_i (J s_j): -2 J with the two spins' signs
+                        const uint32_t v = __float_as_uint(-2.0f * __int_as_float(rn[z].y)) ^ xi ^ xj;
+                        t[z] = real ? v : 0u;
+                        nb[z] = real && j != i ? j : -1;  // its own spin: a field
+                    }
+                    uint32_t tl = 0, tr = 0;
+                    if constexpr (!SA) {
+                        tl = svm2 ^ xi ^ ((sp[i >> 5] >> (i & 31)) << 31);
+                        tr = svm2 ^ xi ^ ((s1[i >> 5] >> (i & 31)) << 31);
+                    }
+                    in = (int)perm[min((b + 1 < nb64 ? (b + 1) * 64 : 0) + lane, N - 1)];
+#pragma unroll
+                    for (int z = 0; z < ZK; ++z) rn[z] = a.rows[(size_t)in * Z + min(z, Z - 1)];
+                    const int cnt = min(64, N - b * 64);
+                    if (!SA && lane == 0) t[0] = __float_as_uint(base + __uint_as_float(t[0]));
+                    auto sum = [&](float x) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int z = 0; z < ZK; ++z) x = x + __uint_as_float(t[z]);
+                        if constexpr (!SA) {
+                            x = x + __uint_as_float(tl);
+                            x = x + __uint_as_float(tr);
+                        }
+                        return x;
+                    };
+                    // Lane q's sum is its terms added to lane q - 1's.  Lanes whose
+                    // sum is right keep it under a further step: the terms of a lane
+                    // change only by flips before its attempt.
+                    float e = SA ? sum(0.0f) : 0.0f;
+                    unsigned long long flips = 0;
+                    int q = 0, npos = 0, want = 4;
+                    auto flip_at = [&](int at) __attribute__((always_inline)) {
+                        flips |= 1ull << at;
+                        const int ia = __builtin_amdgcn_readlane(i, at);
+                        const int iw = lane > at ? ia : -2;
+                        const uint32_t self = i == iw ? 0x80000000u : 0u;  // an order that names a spin twice
+#pragma unroll
+                        for (int z = 0; z < ZK; ++z) t[z] ^= self ^ (nb[z] == iw ? 0x80000000u : 0u);
+                        if constexpr (!SA) {
+                            if (reg != sp) tl ^= self;
+                            if (reg != s1) tr ^= self;
+                        } else {
+                            e = sum(0.0f);
+                        }
+                    };
+                    while (q < cnt) {
+                        // As many attempts as are likely rejected, as if all were:
+                        // attempt q + m then takes output nu + m.
+                        const int len = min(SA ? 64 : want, min(cnt - q, 31 - nu));
+                        const float los = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * (nu + lane - q), __float_as_int(lo)));
+                        if constexpr (!SA)
+                            for (int c = 0; c < len; c += 4) {
+#pragma unroll
+                                for (int y = 0; y < 4; ++y) e = sum(lane_before(e));
+                            }
+                        const unsigned long long open = (__ballot(e >= los) >> q) & ((1ull << len) - 1ull);
+                        const int n = open ? (int)__builtin_ctzll(open) : len;
+                        q += n;
+                        nu += n;
+                        want = 32;
+                        if (n < len) {
+                            want = 4;
+                            float eq = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), q));
+                            if (SA ? eq >= 0.0f : eq > 0.0f) {
+                                // flips without a draw come in runs too
+                                for (;;) {
+                                    ++npos;
+                                    flip_at(q++);
+                                    if (q == cnt) break;
+                                    if constexpr (!SA) e = sum(lane_before(e));
+                                    eq = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), q));
+                                    if (!(SA ? eq >= 0.0f : eq > 0.0f)) break;
+                                }
+                            } else {
+                                bool flip = eq > __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hi), nu));
+                                if (!flip) {
+                                    asm volatile("");  // rare: not to be computed ahead of the branch
+                                    const uint32_t x = (uint32_t)__builtin_amdgcn_readlane((int)rl, nu) >> 1;
+                                    const double u = (double)x / 2147483647.0;
+                                    const double ex = exp((double)(eq / T));
+                                    flip = ex > u;
+                                    if (ex > 0.0 && ex < INFINITY && fabs(ex - u) <= ex * 0x1p-50) ++nt;
+                                }
+                                ++nu;
+                                if (flip) flip_at(q);
+                                ++q;
+                            }
+                        }
+                        if (nu == 31) next_block();
+                    }
+                    base = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), cnt - 1));
+                    nd += (unsigned long long)(cnt - npos);
+                    if ((flips >> lane) & 1ull) atomicXor(reg + (i >> 5), 1u << (i & 31));
+                    sync();
+                }
+                if (own) store(cur, k);
+                sync();
+            }
+        }
+    }
+    if constexpr (SA) {
+        store(cur, 0);
+    } else {
+        store(s1, 1);
+        if (P != 2) store(sp, P - 1);
+    }
+    // the ring as the used outputs leave it
+    if (out) a.rstate[(size_t)r * 32 + slot] = on < nu ? rv : ro;
+    if (lane == 0) {
+        a.rstate[(size_t)r * 32 + 31] = (f0 + (uint32_t)nu) % 31u;
+        a.draws[r] = nd;
+        a.ties[r] = nt;
+    }
+}
+
+// Up to this many replicas in flight at once, a wavefront each beats a lane each.
+// In 1e9 attempts/s, wavefronts against lanes, P=16: 100 spins, 4096 replicas 26.3 to
+// 11.1, 8192 26.0 to 19.5, 16384 26.4 to 33.9; 1024 spins, where the lanes' LDS holds 8192
+// replicas, 2048 17.6 to 6.2 and 16384 29.0 to 12.3.
+constexpr size_t kWaveMaxR = 8192;
+constexpr int kWaveMaxRow = 8;  // couplings of a spin, the widest form built
+
 // int8 [R][P][N] -> bits [P][Wn][R] (bit set = spin -1)
 __global__ void pack_lanes_kernel(const int8_t *confs, uint32_t *bits, int R, int P, int N, int Wn)
 {
@@ -385,7 +664,7 @@ int run_replay(const piqmc_problem *pb, int R, int P, int S, int M, float temp, 
 {
     const int N = pb->N, Wn = (N + 31) / 32;
     const int nreg = sa ? 1 : (P == 2 ? 2 : 3);
-    // Launch shape: W waves per workgroup share one LDS copy of the neighbour
+    // Launch shape, a lane each: W waves per workgroup share one LDS copy of the neighbour
     // rows; Lw lanes per wave each own a replica.  Lw is the smallest power of
     // two that still gives every CU two workgroups, so replicas spread over all
     // SIMDs with two chains' latency to hide per SIMD (4096 replicas of the
@@ -445,18 +724,36 @@ int run_replay(const piqmc_problem *pb, int R, int P, int S, int M, float temp, 
     a.draws = d_draws;
     a.ties = ties;
     a.jd = pb->dense ? pb->d_jd : nullptr;
-    // the AND-OR neighbour address needs slot offsets below 32 bytes
-    const bool ora = staged && !pb->dense && L <= 8;
-    auto pick = [&](auto SAc) {
-        constexpr bool S_ = decltype(SAc)::value;
-        return pb->dense ? (staged ? replay_kernel<true, true, S_> : replay_kernel<true, false, S_>)
-                         : (staged ? (ora ? replay_kernel<false, true, S_, true> : replay_kernel<false, true, S_>)
-                                   : replay_kernel<false, false, S_>);
-    };
-    auto kern = sa ? pick(std::true_type()) : pick(std::false_type());
-    (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds(L));
-    piqmc::timing_begin(st);
-    kern<<<(R + L - 1) / L, 64 * W, lds(L), st>>>(a);
+    // a wavefront per replica: as many per workgroup as the LDS holds
+    int ww = 4;
+    auto wlds = [&] { return (size_t)ww * replay_wave_words(N, Wn, sa) * 4; };
+    while (ww > 1 && wlds() > kLds) ww /= 2;
+    const size_t lanes = std::min((size_t)R, kLds / lds(L) * L * kCUs);  // replicas in flight, a lane each
+    if (!pb->dense && pb->Z <= kWaveMaxRow && lanes <= kWaveMaxR && wlds() <= kLds) {
+        auto pickw = [&](auto SAc) {
+            constexpr bool S_ = decltype(SAc)::value;
+            return pb->Z <= 4 ? replay_wave_kernel<S_, 4>
+                              : (pb->Z <= 5 ? replay_wave_kernel<S_, 5>
+                                            : (pb->Z <= 6 ? replay_wave_kernel<S_, 6> : replay_wave_kernel<S_, 8>));
+        };
+        auto kern = sa ? pickw(std::true_type()) : pickw(std::false_type());
+        (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wlds());
+        piqmc::timing_begin(st);
+        kern<<<(R + ww - 1) / ww, 64 * ww, wlds(), st>>>(a);
+    } else {
+        // the AND-OR neighbour address needs slot offsets below 32 bytes
+        const bool ora = staged && !pb->dense && L <= 8;
+        auto pick = [&](auto SAc) {
+            constexpr bool S_ = decltype(SAc)::value;
+            return pb->dense ? (staged ? replay_kernel<true, true, S_> : replay_kernel<true, false, S_>)
+                             : (staged ? (ora ? replay_kernel<false, true, S_, true> : replay_kernel<false, true, S_>)
+                                       : replay_kernel<false, false, S_>);
+        };
+        auto kern = sa ? pick(std::true_type()) : pick(std::false_type());
+        (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds(L));
+        piqmc::timing_begin(st);
+        kern<<<(R + L - 1) / L, 64 * W, lds(L), st>>>(a);
+    }
     piqmc::timing_end(st);
     PIQMC_HIP(hipGetLastError());
     unpack_lanes_kernel<<<grid_for((size_t)R * P * N, 256), 256, 0, st>>>(d_bits, confs, R, P, N, Wn);
