@@ -118,19 +118,34 @@ __device__ T block_sum(T v, T *red)
     return t;
 }
 
-// Three-input XOR and majority of bit-sliced words (one gfx950 v_bitop3_b32
-// each for 32-bit words: truth tables 0x96 and 0xE8, symmetric in the inputs).
+// Three-input logic of bit-sliced words, one gfx950 v_bitop3_b32 for each 32-bit
+// half (the compiler forms none from plain operators).  TT is the truth table
+// over (a, b, c) = (0xF0, 0xCC, 0xAA).
+template <int TT, typename WT>
+__device__ __forceinline__ WT bop(WT a, WT b, WT c)
+{
+    if constexpr (sizeof(WT) == 4) {
+        return __builtin_amdgcn_bitop3_b32(a, b, c, TT);
+    } else {
+        return (WT)bop<TT, uint32_t>((uint32_t)a, (uint32_t)b, (uint32_t)c) |
+               ((WT)bop<TT, uint32_t>((uint32_t)(a >> 32), (uint32_t)(b >> 32), (uint32_t)(c >> 32)) << 32);
+    }
+}
 template <typename WT>
 __device__ __forceinline__ WT xor3(WT a, WT b, WT c)
 {
-    if constexpr (sizeof(WT) == 4) return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
-    else return a ^ b ^ c;
+    return bop<0x96, WT>(a, b, c);
 }
 template <typename WT>
 __device__ __forceinline__ WT maj3(WT a, WT b, WT c)
 {
-    if constexpr (sizeof(WT) == 4) return __builtin_amdgcn_bitop3_b32(a, b, c, 0xE8);
-    else return (a & b) | (c & (a ^ b));
+    return bop<0xE8, WT>(a, b, c);
+}
+// c ? a : b, bit by bit
+template <typename WT>
+__device__ __forceinline__ WT sel3(WT c, WT a, WT b)
+{
+    return bop<0xCA, WT>(c, a, b);
 }
 
 // t-th bit-sliced random word of a Philox4x32 output block: four 32-bit words
@@ -594,6 +609,12 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
     #pragma unroll(FIXED ? kFixRep : 1)
                             for (int rr = 0; rr < nrep; ++rr) {
                               WT qX = 0, qm0 = 0, qm1 = 0, qm2 = 0;  // stochastic word for the queue
+                              uint32_t inf = info;
+                              if constexpr (FLD) {
+                                  // formed here: hoisted out of this loop, the masks of these
+                                  // bits would hold (and spill) scalar register pairs
+                                  asm volatile("" : "+v"(inf), "+v"(fc.ka), "+v"(fc.ks));
+                              }
                               if (act) {
                                 WT *mine = st + ((size_t)rr * 2 + tau) * PW;
                                 const WT *other = st + ((size_t)rr * 2 + 1 - tau) * PW;
@@ -614,7 +635,7 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                         WT x[ZU];
     #pragma unroll
                                         for (int z = 0; z < ZU; ++z)
-                                            x[z] = xor3<WT>(S_, nbword(mine, nb[z]), ((info >> z) & 1u) ? ~WT(0) : WT(0));
+                                            x[z] = xor3<WT>(S_, nbword(mine, nb[z]), FLD ? bitmask<WT>(inf, z) : (((inf >> z) & 1u) ? ~WT(0) : WT(0)));
                                         if constexpr (ZU == 4) {
                                             const WT s1 = xor3<WT>(x[0], x[1], x[2]), k1 = maj3<WT>(x[0], x[1], x[2]);
                                             c0 = s1 ^ x[3];
@@ -633,7 +654,7 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
     #pragma unroll
                                     for (int z = 0; z < 8; ++z) {
                                         if (ZU > 0 ? z < ZU : (z < a.zmax && z < zi)) {
-                                            const WT x = S_ ^ nbword(mine, nb[z]) ^ (((info >> z) & 1u) ? ~WT(0) : WT(0));
+                                            const WT x = S_ ^ nbword(mine, nb[z]) ^ (((inf >> z) & 1u) ? ~WT(0) : WT(0));
                                             const WT k0 = c0 & x;
                                             c0 ^= x;
                                             const WT k1 = c1 & k0;
@@ -644,6 +665,7 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                     }
                                     // Trotter classes; bits past W are zero in every class
                                     const WT e0 = ~(uL | uR) & valid, e1 = uL ^ uR, e2 = uL & uR;
+                                    const WT xr = FLD ? WT(Lw ^ Rw) : WT(0);  // exactly one antiparallel Trotter bond
                                     WT X;
                                     WT ge[KMAX + 1];  // "count >= k" masks (uniform-degree path)
                                     if (FLD) {
@@ -652,22 +674,27 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                         // bit planes by selects on (S_, uL, uR) -- u_t = 1 where uL
                                         // and uR differ, else 2 or 0 by uL -- and compared with the
                                         // bond count once: the same masks as a "count >= k" per
-                                        // (sigma, u_t) class, in a third of the work.
-                                        const WT xr = uL ^ uR;
+                                        // (sigma, u_t) class, in a third of the work.  As three-input
+                                        // operations on masks formed per word: 398 -> 197 VALU
+                                        // instructions a 64-bit word before its draws, and 92 -> 76 a
+                                        // Philox block of them (12^3 lattice, P=128, 1024 replicas, 100
+                                        // sweeps: 12.9 -> 9.4 ms).
                                         auto kplane = [&](uint32_t pk, int j) __attribute__((always_inline)) -> WT {
                                             const WT a0 = bitmask<WT>(pk, j), a1 = bitmask<WT>(pk, 4 + j),
                                                      a2 = bitmask<WT>(pk, 8 + j);
                                             const WT b0 = bitmask<WT>(pk, 12 + j), b1 = bitmask<WT>(pk, 16 + j),
                                                      b2 = bitmask<WT>(pk, 20 + j);
-                                            const WT fp = (xr & a1) | (~xr & ((uL & a2) | (~uL & a0)));
-                                            const WT fn = (xr & b1) | (~xr & ((uL & b2) | (~uL & b0)));
-                                            return (S_ & fn) | (~S_ & fp);
+                                            return sel3<WT>(S_, sel3<WT>(xr, b1, sel3<WT>(uL, b2, b0)),
+                                                            sel3<WT>(xr, a1, sel3<WT>(uL, a2, a0)));
+                                        };
+                                        // (c & ~K) | (~(c ^ K) & t) per plane: the majority of c, ~K and t
+                                        auto step = [](WT c, WT K, WT t) __attribute__((always_inline)) -> WT {
+                                            return bop<0xB2, WT>(c, K, t);
                                         };
                                         auto ge_k = [&](uint32_t pk) __attribute__((always_inline)) -> WT {
-                                            const WT K0 = kplane(pk, 0), K1 = kplane(pk, 1), K2 = kplane(pk, 2);
-                                            WT t = c0 | ~K0;
-                                            t = (c1 & ~K1) | (~(c1 ^ K1) & t);
-                                            t = (c2 & ~K2) | (~(c2 ^ K2) & t);
+                                            WT t = c0 | ~kplane(pk, 0);
+                                            t = step(c1, kplane(pk, 1), t);
+                                            t = step(c2, kplane(pk, 2), t);
                                             // thresholds reach 8 ("never") only with seven couplings
                                             if constexpr (!(ZU > 0 && ZU <= 6)) t &= ~kplane(pk, 3);
                                             return t;
@@ -754,11 +781,17 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                                 if (t < ns) {
                                                     const uint32_t sb = (fc.slot >> (8 * t)) & 255u;
                                                     const int cb = (int)(sb & 7u);
-                                                    const WT eu = (cb % 3) == 0 ? e0 : ((cb % 3) == 1 ? e1 : e2);
+                                                    // bits that are not of the triple: another sign, another
+                                                    // u_t (1 where xr, else 2 or 0 by uL) or another count
+                                                    const uint32_t ut = (uint32_t)(cb % 3);
+                                                    const WT m1 = bitmask<WT>(ut, 0), m2 = bitmask<WT>(ut, 1);
+                                                    WT ne = (xr ^ m1) | (uL & ~xr & ~m2) | (~uL & m2);
+                                                    ne |= S_ ^ (cb < 3 ? WT(0) : ~WT(0));
                                                     // count == u_s (u_s <= 7: three bits at 4..6 of the slot)
-                                                    const WT eq = ~((c0 ^ bitmask<WT>(sb, 4)) | (c1 ^ bitmask<WT>(sb, 5)) |
-                                                                    (c2 ^ bitmask<WT>(sb, 6)));
-                                                    const WT mk = (cb < 3 ? ~S_ : S_) & eu & eq;
+                                                    ne = bop<0xF6, WT>(ne, c0, bitmask<WT>(sb, 4));
+                                                    ne = bop<0xF6, WT>(ne, c1, bitmask<WT>(sb, 5));
+                                                    ne = bop<0xF6, WT>(ne, c2, bitmask<WT>(sb, 6));
+                                                    const WT mk = X & ~ne;
                                                     if (t == 0) { cm0 = mk; ct0 = fc.st[0]; }
                                                     else if (t == 1) { cm1 = mk; ct1 = fc.st[1]; }
                                                     else { cm2 = mk; ct2 = fc.st[2]; }
@@ -819,8 +852,9 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                                 WT tb;  // bits whose class threshold has bit sh set
                                                 // (with fields more than three classes never get here)
                                                 if (FLD || ns <= 3) {
-                                                    tb = (((ct0 >> sh) & 1u) ? cm0 : WT(0)) | (((ct1 >> sh) & 1u) ? cm1 : WT(0)) |
-                                                         (((ct2 >> sh) & 1u) ? cm2 : WT(0));
+                                                    // a | (b & c)
+                                                    tb = bop<0xF8, WT>(bop<0xF8, WT>(cm0 & bitmask<WT>(ct0, sh), cm1, bitmask<WT>(ct1, sh)),
+                                                                       cm2, bitmask<WT>(ct2, sh));
                                                 } else {
                                                     tb = 0;
     #pragma unroll
@@ -832,8 +866,8 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                                                 tb |= eu & ge_pick(us, c0, c1, c2) & ~ge_pick(us + 1, c0, c1, c2);
                                                     }
                                                 }
-                                                lt |= und & ~Rb & tb;
-                                                und &= ~(Rb ^ tb);
+                                                lt |= bop<0x20, WT>(und, Rb, tb);   // und & ~Rb & tb
+                                                und = bop<0x90, WT>(und, Rb, tb);   // und & ~(Rb ^ tb)
                                             }
                                         }
                                         flips |= lt & X;
