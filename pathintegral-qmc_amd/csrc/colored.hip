@@ -228,7 +228,13 @@ __device__ __forceinline__ void field_classes(double h, int z, float jp, double 
         while (amin > 0 && Xat(amin - 1) < 0.0) --amin;
         int smin, us = amin - 1;
         unsigned int thr = 0;
-        int cls = us >= 0 ? field_class(hs, z, us, B, T, &thr) : 1;
+        int cls = us >= 0 ? field_class(hs, z, us, B, T, &thr) : 0;
+        // no energy change, or so little that every draw accepts: a bit without a
+        // field whose bonds balance
+        while (cls == 1) {
+            amin = us--;
+            cls = us >= 0 ? field_class(hs, z, us, B, T, &thr) : 0;
+        }
         smin = amin;
         for (; us >= 0 && cls == 2; --us) {
             smin = us;
