@@ -183,6 +183,24 @@ __device__ __forceinline__ WT bitmask(uint32_t pk, int bit)
     return (WT)(int64_t)((int32_t)(pk << (31 - bit)) >> 31);  // 0 or all ones
 }
 
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The cached field sweep's queue of open bits: entries per wavefront (at most
+// 63 + 64 held), and the Philox blocks a word's draws take in line before it.
+// Few bits need more, but some lane of 64 nearly always has one: about six blocks
+// ran for a wavefront's words where 2.3 decide the average word.  Four bits of
+// every uniform in line for 32-bit words, six for 64-bit ones (12^3 lattice, a
+// sweep of 4 replicas: P=64 11.3 us, eight bits 12.2; P=128 18.4 us, four bits 19.4,
+// eight 19.6; without the queue 12.4 and 20.1).
+constexpr int kFieldCap = 128;
+template <typename WT>
+constexpr int kFieldAhead = sizeof(WT) == 4 ? 1 : 3;
+
 // Decision classes of one spin with a field h in one field step, for +-1
 // couplings: a bit's class depends only on its spin's sign sigma, its
 // unsatisfied-bond count u_s (0..z) and antiparallel Trotter bonds u_t, via
@@ -319,6 +337,10 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
     uint4 *wq = reinterpret_cast<uint4 *>(wqb);           // several classes
     uint2 *wq1 = reinterpret_cast<uint2 *>(wqb);          // single class: fresh words
     uint4 *wq2 = reinterpret_cast<uint4 *>(wqb + 8 * kQueueCap1);  // single class: undecided after block 0
+    // open bits of the cached field sweep (FQ): spin | bit << 16 | parity << 22 |
+    // replica << 23, and the bit's draw threshold
+    constexpr bool FQ = FLD && CACHED;
+    uint2 *fq = reinterpret_cast<uint2 *>(red + 16) + (tid >> 6) * kFieldCap;
     int qn = 0;  // queued records of this wavefront (wave-uniform)
     int q2 = 0;  // records in wq2 (wave-uniform)
     const WT valid = (W == (int)(8 * sizeof(WT))) ? ~WT(0) : ((WT(1) << W) - 1);
@@ -421,14 +443,14 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
         const float jp = a.jperp[s];
         const double Ts = (double)a.temps[s];
         // cached spins with fields: their decision classes of this field step
-        FieldClasses cfc[2][2];
+        FieldClasses cfc[2][2] = {};
         if constexpr (FLD && CACHED) {
 #pragma unroll
             for (int c = 0; c < 2; ++c)
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
                     const int q = c == 0 ? (k == 0 ? cq_[0][0] : cq_[0][1]) : (k == 0 ? cq_[1][0] : cq_[1][1]);
-                    field_classes(q >= 0 ? (double)a.hq[q] : 0.0, ZU, jp, Ts, cfc[c][k]);
+                    if (q >= 0) field_classes((double)a.hq[q], ZU, jp, Ts, cfc[c][k]);
                 }
         }
         const bool cq = CQ && un <= 3;  // this step's stochastic words go through the queue
@@ -611,6 +633,54 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                         qn -= cnt;
                         __builtin_amdgcn_wave_barrier();
                     };
+                    // The last cnt open bits of the field sweep: what the Philox blocks
+                    // computed in line (kFieldAhead) left undecided, a lane each, or
+                    // four lanes with a block each where at most 16 are left.
+                    auto drain_bits = [&](const int cnt) __attribute__((always_inline)) {
+                        constexpr int kPer = sizeof(WT) == 4 ? 4 : 2;
+                        wave_sync();
+                        const int lane = tid & 63, sh4 = cnt <= 16 ? 2 : 0, e = lane >> sh4;
+                        const bool on = e < cnt;
+                        const uint2 en = fq[qn - cnt + (on ? e : 0)];
+                        const int ei = (int)(en.x & 0xffffu), m = (int)((en.x >> 16) & 63u);
+                        const int et = (int)((en.x >> 22) & 1u), er = (int)(en.x >> 23);
+                        const uint32_t rep = a.replica_base + (uint32_t)(r0 + er);
+                        int qd = kFieldAhead<WT> + (sh4 ? (lane & 3) : 0);
+                        bool open = on, less = false;
+                        do {
+                            // kPer bits of the uniform against the threshold's, as numbers
+                            uint32_t o[4], v = 0;
+                            philox4x32_10(g, (uint32_t)ei, rep, ((uint32_t)et << 24) | (uint32_t)qd, a.key0, a.key1, o);
+#pragma unroll
+                            for (int t = 0; t < kPer; ++t) {
+                                const uint32_t w = sizeof(WT) == 4 ? o[t] : (m < 32 ? o[2 * t] : o[(2 * t + 1) & 3]);
+                                v = (v << 1) | ((w >> (m & 31)) & 1u);
+                            }
+                            const bool past = qd >= 32 / kPer;  // all 32 bits equal: not below
+                            const uint32_t tv = past ? 0u : (en.y >> (32 - kPer * (qd + 1))) & ((1u << kPer) - 1u);
+                            const bool lt = !past && v < tv, ne = past || v != tv;
+                            if (sh4) {
+                                // the entry's first block that differs decides
+                                const uint32_t nq = (uint32_t)(__ballot(ne) >> (lane & ~3)) & 15u;
+                                const uint32_t lq = (uint32_t)(__ballot(lt) >> (lane & ~3)) & 15u;
+                                if (open && nq) {
+                                    less = ((lq >> (__ffs(nq) - 1)) & 1u) != 0u;
+                                    open = false;
+                                }
+                                qd += 4;
+                            } else {
+                                if (open && ne) {
+                                    less = lt;
+                                    open = false;
+                                }
+                                ++qd;
+                            }
+                        } while (__ballot(open));
+                        if (on && less && (sh4 == 0 || (lane & 3) == 0))
+                            atomicXor(reinterpret_cast<uint32_t *>(st + ((size_t)er * 2 + et) * PW + ei) + (m >> 5), 1u << (m & 31));
+                        qn -= cnt;
+                        wave_sync();
+                    };
                     // one spin (position q in color order, index i, neighbours nb)
                     // for every replica of the workgroup; lanes with act false take
                     // part only in the queue's wave-wide steps
@@ -622,17 +692,16 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                             const uint32_t zt = UZ ? zt_u : ((PMJ && !FLD) ? tz[zi] : 0u);
                             // fields: this spin's class thresholds, shared by the replicas below
                             // (cached spins: computed once per field step)
-                            double hfield = 0.0;
                             FieldClasses fc;
                             if (FLD) {
-                                hfield = (double)a.hq[q];
                                 if (fcp) fc = *fcp;
-                                else field_classes(hfield, zi, jp, Ts, fc);
+                                else field_classes((double)a.hq[q], zi, jp, Ts, fc);
                             }
                             // fixed planes: unrolled, so each replica's planes are immediates
     #pragma unroll(FIXED ? kFixRep : 1)
                             for (int rr = 0; rr < nrep; ++rr) {
                               WT qX = 0, qm0 = 0, qm1 = 0, qm2 = 0;  // stochastic word for the queue
+                              WT fX = 0, fm0 = 0, fm1 = 0;           // open bits (FQ), and of the first two triples
                               uint32_t inf = info;
                               if constexpr (FLD) {
                                   // formed here: hoisted out of this loop, the masks of these
@@ -843,6 +912,7 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                             // (out of line as a called function it costs more in the
                                             // call's register traffic than it saves: 297 -> 301 ms
                                             // on the 3-D L=12 field workload)
+                                            const double hfield = (double)a.hq[q];
                                             for (int mm = 0; mm < W; ++mm) {
                                                 if (!((X >> mm) & WT(1))) continue;
                                                 const int sg = (int)((S_ >> mm) & WT(1));
@@ -865,7 +935,7 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                             }
                                             und = 0;
                                         }
-                                        for (int qd = 0; qd < 32 / kPer && und; ++qd) {
+                                        for (int qd = 0; qd < (FQ ? kFieldAhead<WT> : 32 / kPer) && und; ++qd) {
                                             uint32_t out[4];
                                             philox4x32_10(g, (uint32_t)i, rep, (uint32_t(tau) << 24) | (uint32_t)qd,
                                                           a.key0, a.key1, out);
@@ -895,6 +965,11 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                             }
                                         }
                                         flips |= lt & X;
+                                        if constexpr (FQ) {
+                                            fX = und;
+                                            fm0 = cm0;
+                                            fm1 = cm1;
+                                        }
                                     }
                                 } else {
                                     const int2 *row = a.rows + (size_t)i * a.Z;
@@ -937,6 +1012,24 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                     }
                                 }
                                 mine[i] = S_ ^ flips;
+                              }
+                              if constexpr (FQ) {
+                                  while (__ballot(fX != 0)) {
+                                      const bool has = fX != 0;
+                                      const unsigned long long bal = __ballot(has);
+                                      if (has) {
+                                          const int m = __ffsll((unsigned long long)fX) - 1;
+                                          fX &= fX - 1;
+                                          const uint32_t th = (fm0 >> m) & 1 ? fc.st[0] : ((fm1 >> m) & 1 ? fc.st[1] : fc.st[2]);
+                                          const int pos = qn + (int)__builtin_amdgcn_mbcnt_hi(
+                                                                   (uint32_t)(bal >> 32),
+                                                                   __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+                                          fq[pos] = make_uint2((uint32_t)i | ((uint32_t)m << 16) | ((uint32_t)tau << 22) |
+                                                                   ((uint32_t)rr << 23), th);
+                                      }
+                                      qn += (int)__popcll(bal);
+                                      if (qn >= 64) drain_bits(64);
+                                  }
                               }
                               if constexpr (CQ && !DET) {
                                   if (cqm) {
@@ -986,7 +1079,7 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                             constexpr int tp = ph == 0 ? 0 : (ph == 2 ? 1 : part);
                             constexpr int c = ph == 0 ? 0 : (ph == 2 ? 1 : 1 - part);
                             const int q = cq_[c][k];
-                            if (!CQ && q < 0) return;
+                            if (!CQ && !FQ && q < 0) return;
                             int nb[ZC];
     #pragma unroll
                             for (int z = 0; z < ZC; ++z) nb[z] = cN[c][k][z];
@@ -1021,6 +1114,9 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
                                 if (qn + q2 > 0) drain_last();
                             } else if (CQ && !DET && qn > 0) {
                                 drain(qn, std::integral_constant<int, 3>());
+                            }
+                            if constexpr (FQ) {
+                                if (qn > 0) drain_bits(qn);
                             }
                             __syncthreads();
                         };
@@ -1123,14 +1219,14 @@ __global__ void __attribute__((flatten)) colored_kernel(ColArgs<WT> a)
     colored_body<WT, PMJ, UZ, FLD, ZU, CACHED, CQ>(a, r0, min(a.rpw, a.R - r0), smem);
 }
 
-// The field sweep with cached spins and decision classes (cubic lattices): at
+// The field sweep with cached spins and decision classes (square and cubic lattices): at
 // most 512 threads, so that the cached registers fit without spilling.
-template <typename WT>
+template <typename WT, int ZU>
 __global__ void __attribute__((flatten)) __launch_bounds__(512) colored_fields_cached_kernel(ColArgs<WT> a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const int r0 = blockIdx.x * a.rpw;
-    colored_body<WT, true, false, true, 6, true, false>(a, r0, min(a.rpw, a.R - r0), smem);
+    colored_body<WT, true, false, true, ZU, true, false>(a, r0, min(a.rpw, a.R - r0), smem);
 }
 
 // The queue kernels (+-1 couplings, uniform degree) with a register budget of
@@ -2724,7 +2820,9 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
     // per-bit general path
     const SparseTile tile = sparse_tile(pb, R, sizeof(WT), block, rpw, chains);
     const bool sparse = tile.block > 0;
-    if (rpw <= 0 && pb->pmjf && !pb->pmj && pb->ncolors == 2 && pb->zuni_nf == 6 && cached_fields_enabled()) {
+    const bool cached_fields = pb->pmjf && !pb->pmj && pb->ncolors == 2 && (pb->zuni_nf == 4 || pb->zuni_nf == 6) &&
+                               cached_fields_enabled();
+    if (rpw <= 0 && cached_fields) {
         // the cached field sweep evaluates each step's decision classes once per
         // workgroup for all of its replicas: as many replicas per workgroup as
         // put every workgroup on the device at once (one 512-thread workgroup
@@ -2734,7 +2832,8 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
             ncu = 256;
-        const size_t per = sizeof(WT) * 2 * (size_t)N, fixed_part = 4 * (kClassStride + 8) + 16 * sizeof(double);
+        const size_t per = sizeof(WT) * 2 * (size_t)N;
+        const size_t fixed_part = 4 * (kClassStride + 8) + 16 * sizeof(double) + (size_t)8 * kFieldCap * sizeof(uint2);
         const int lds_max = (int)std::max<size_t>(1, (160 * 1024 - fixed_part) / per);
         rpw = std::max(1, std::min(lds_max, (R + ncu - 1) / ncu));
     }
@@ -2800,13 +2899,14 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         a.zuni = -1;
         int biggest = 0;
         for (int c = 0; c < pb->ncolors; ++c) biggest = std::max(biggest, pb->color_off[c + 1] - pb->color_off[c]);
-        // two colors of at most two spins per thread and six couplings per
-        // spin besides the field (cubic lattices): spins, neighbours and
-        // decision classes cached in registers
-        if (pb->ncolors == 2 && biggest <= 2 * block && block <= 512 && pb->zuni_nf == 6 && cached_fields_enabled()) {
-            (void)hipFuncSetAttribute((const void *)colored_fields_cached_kernel<WT>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            colored_fields_cached_kernel<WT><<<grid, block, lds, st>>>(a);
+        // two colors of at most two spins per thread and four or six couplings
+        // per spin besides the field (square and cubic lattices): spins,
+        // neighbours and decision classes cached in registers
+        const size_t lf = lds + (size_t)(block / 64) * kFieldCap * sizeof(uint2);
+        if (biggest <= 2 * block && block <= 512 && lf <= 160 * 1024 && cached_fields) {
+            auto kern = pb->zuni_nf == 4 ? colored_fields_cached_kernel<WT, 4> : colored_fields_cached_kernel<WT, 6>;
+            (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lf);
+            kern<<<grid, block, lf, st>>>(a);
         } else {
             (void)hipFuncSetAttribute((const void *)colored_kernel<WT, true, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             colored_kernel<WT, true, false, true><<<grid, block, lds, st>>>(a);
