@@ -24,6 +24,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <initializer_list>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -2639,6 +2640,33 @@ struct CallBuffers {
     }
 };
 
+// The host tables of a call, uploaded as one buffer by one copy: each further
+// allocation and copy of a small call costs the host more than the tables' bytes
+// (64 spins, one replica, 100 steps: 426 us with a copy each, 417 so).  Each table
+// begins at a multiple of 256 bytes.
+struct Table {
+    const void *src;  // null: room only
+    size_t bytes;
+    void **dst;
+};
+int upload_tables(CallBuffers &buf, std::initializer_list<Table> tables)
+{
+    size_t total = 0;
+    for (const Table &t : tables) total += CallBuffers::round_up(t.bytes);
+    unsigned char *base = nullptr;
+    int rc = buf.take((void **)&base, total);
+    if (rc) return rc;
+    std::vector<unsigned char> host(total);
+    size_t at = 0;
+    for (const Table &t : tables) {
+        if (t.src && t.bytes) std::memcpy(host.data() + at, t.src, t.bytes);
+        *t.dst = base + at;
+        at += CallBuffers::round_up(t.bytes);
+    }
+    PIQMC_HIP(hipMemcpyAsync(base, host.data(), total, hipMemcpyHostToDevice, buf.st));
+    return PIQMC_OK;
+}
+
 // Device bytes a parallel-sweep call takes from a CallBuffers region (each
 // buffer rounded up to 256 bytes): J_perp and temperatures [2S] floats, the
 // +-1 path's per-step tables, the color offsets and the packed state
@@ -2752,9 +2780,9 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         float *d_jp = nullptr;  // [S] J_perp, then [S] temperatures
         WT *d_packed = nullptr;
         double *d_fields = nullptr;
-        if ((rc = buf.take((void **)&d_jp, sizeof(float) * (S ? 2 * S : 1)))) return rc;
-        if (S) PIQMC_HIP(hipMemcpyAsync(d_jp, jp.data(), sizeof(float) * S, hipMemcpyHostToDevice, st));
-        if (S) PIQMC_HIP(hipMemcpyAsync(d_jp + S, temps.data(), sizeof(float) * S, hipMemcpyHostToDevice, st));
+        std::vector<float> jt(jp);
+        jt.insert(jt.end(), temps.begin(), temps.end());
+        if ((rc = upload_tables(buf, {{jt.data(), sizeof(float) * 2 * S, (void **)&d_jp}}))) return rc;
         if ((rc = buf.take((void **)&d_packed, sizeof(WT) * 2 * (size_t)N * R))) return rc;
         if (fields && (rc = buf.take((void **)&d_fields, sizeof(double) * 2 * (size_t)W * fields_pitch(N) * R)))
             return rc;
@@ -2826,8 +2854,8 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         // the cached field sweep evaluates each step's decision classes once per
         // workgroup for all of its replicas: as many replicas per workgroup as
         // put every workgroup on the device at once (one 512-thread workgroup
-        // per CU), within the LDS (3-D L=12 field workload, 1024 replicas: 4
-        // per workgroup 251 ms, 2 298 ms, 3 400 ms, 1 392 ms)
+        // per CU), within the LDS (12^3 lattice with fields, P=128, 1024
+        // replicas, 100 sweeps: 4 per workgroup 8.3 ms, 2 9.6, 3 13.0, 1 12.0)
         int dev = 0, ncu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
@@ -2862,21 +2890,16 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
     uint32_t *d_thr = nullptr, *d_zt = nullptr;
     int *d_coff = nullptr;
     WT *d_packed = nullptr;
-    if ((rc = buf.take((void **)&d_jp, sizeof(float) * (S ? 2 * S : 1)))) return rc;
-    if (S) PIQMC_HIP(hipMemcpyAsync(d_jp, jp.data(), sizeof(float) * S, hipMemcpyHostToDevice, st));
-    if (S) PIQMC_HIP(hipMemcpyAsync(d_jp + S, temps.data(), sizeof(float) * S, hipMemcpyHostToDevice, st));
-    if (pb->pmj && S) {
-        // taken whenever the problem is +-1 (as colored_scratch_bytes counts),
-        // filled only when the tables apply
-        if ((rc = buf.take((void **)&d_thr, sizeof(uint32_t) * (size_t)S * kClassStride))) return rc;
-        if ((rc = buf.take((void **)&d_zt, sizeof(uint32_t) * (size_t)S * 8))) return rc;
-        if (pmj) {
-            PIQMC_HIP(hipMemcpyAsync(d_thr, thr.data(), sizeof(uint32_t) * thr.size(), hipMemcpyHostToDevice, st));
-            PIQMC_HIP(hipMemcpyAsync(d_zt, ztab.data(), sizeof(uint32_t) * ztab.size(), hipMemcpyHostToDevice, st));
-        }
-    }
-    if ((rc = buf.take((void **)&d_coff, sizeof(int) * (pb->ncolors + 1)))) return rc;
-    PIQMC_HIP(hipMemcpyAsync(d_coff, pb->color_off.data(), sizeof(int) * (pb->ncolors + 1), hipMemcpyHostToDevice, st));
+    std::vector<float> jt(jp);
+    jt.insert(jt.end(), temps.begin(), temps.end());
+    // the +-1 tables' room is taken whenever the problem is +-1 (as
+    // colored_scratch_bytes counts), filled only when the tables apply
+    const size_t nt = pb->pmj ? sizeof(uint32_t) * (size_t)S : 0;
+    if ((rc = upload_tables(buf, {{jt.data(), sizeof(float) * 2 * S, (void **)&d_jp},
+                                  {pb->color_off.data(), sizeof(int) * (pb->ncolors + 1), (void **)&d_coff},
+                                  {pmj ? ztab.data() : nullptr, nt * 8, (void **)&d_zt},
+                                  {pmj ? thr.data() : nullptr, nt * kClassStride, (void **)&d_thr}})))
+        return rc;
     if ((rc = buf.take((void **)&d_packed, sizeof(WT) * 2 * (size_t)N * R))) return rc;
     launch_pack<WT>(confs, d_packed, R, P, N, st);
 
