@@ -2884,6 +2884,22 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         int biggest = 0;
         for (int c = 0; c < pb->ncolors; ++c) biggest = std::max(biggest, pb->color_off[c + 1] - pb->color_off[c]);
         block = biggest > 512 ? 512 : 256;
+        if (pmj && pb->zuni >= 0) {
+            if (pb->ncolors == 2) {
+                // 1024 where that keeps two spins a thread, so that neighbours stay
+                // in registers (64 x 64, P=40: 4 replicas, 40 steps 589 -> 406 us; 512
+                // replicas, 20 steps 498 -> 454), and the queues still fit
+                if (biggest > 1024 && biggest <= 2048 && queue_lds(N, rpw, sizeof(WT), 1024) <= 160 * 1024) block = 1024;
+            } else {
+                // more colors reload their neighbours: with a workgroup a CU, 512
+                // threads for the latency of a class's passes (25 x 25, P=100, 200
+                // replicas 739 -> 643 us; 9^3, P=64, 100 replicas 474 -> 432); with
+                // several, 256 for the draws' partial batches a wavefront ends
+                // each phase with (33 x 33, P=50: 301 replicas 1655 -> 1572 us, 2000
+                // 1435 -> 1264; 11^3, P=64, 800 replicas 757 -> 664)
+                block = biggest > 256 && (R + rpw - 1) / rpw <= 256 ? 512 : 256;
+            }
+        }
     }
     if (block > 1024 || (block & 63)) return piqmc::set_error(PIQMC_EINVAL, "block must be a multiple of 64, <= 1024");
     float *d_jp = nullptr;  // [S] J_perp, then [S] temperatures
