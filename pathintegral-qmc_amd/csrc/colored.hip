@@ -1181,6 +1181,26 @@ __device__ void colored_body(const ColArgs<WT> &a, int r0, int nrep_, unsigned c
             for (int rr = 0; rr < nrep; ++rr) {
                 const WT *s0 = st + (size_t)rr * 2 * PW, *s1 = s0 + PW;
                 double acc = 0.0;
+                if constexpr (PMJ && UZ && !FLD && !FIXED) {
+                    // +-1 couplings only: a whole number of halves, from the color-ordered
+                    // neighbours (at most 20480 spins x 7 x 128; 33 x 33, P=50, 301
+                    // replicas, 60 traced steps: 1.84 -> 1.51 ms against the double rows)
+                    int h = 0;
+                    const int zn = ZU > 0 ? ZU : a.zuni;
+                    for (int q = tid; q < N; q += bd) {
+                        const int i = a.order[q];
+                        const uint32_t info = a.cinfo[q];
+                        const WT a0 = s0[i], a1 = s1[i];
+#pragma unroll
+                        for (int z = 0; z < (ZU > 0 ? ZU : 7); ++z) {
+                            if (z >= zn) break;
+                            const int j = a.cnb[(size_t)z * N + q];
+                            const int sm = a.P - 2 * (popc(a0 ^ s0[j]) + popc(a1 ^ s1[j]));
+                            h += ((info >> z) & 1u) ? sm : -sm;
+                        }
+                    }
+                    acc = 0.5 * (double)h;
+                } else
                 for (int i = tid; i < N; i += bd) {
                     const WT a0 = s0[i], a1 = s1[i];
                     const int2 *row = a.rows + (size_t)i * a.Z;
