@@ -86,9 +86,11 @@ int piqmc_problem_set_sweep_path(piqmc_problem *pb, int path);
  * slice; 2 each slice's field split over 64/(P/2) lanes; 3 one replica per
  * workgroup of four wavefronts (the field split over them); 4 / 5 that
  * workgroup pipelined, one wavefront deciding a spin while three / seven sum
- * the next one's field; 6 one replica per wavefront with every spin's local
- * field in every slice of the swept parity kept in LDS and updated on flips
- * (rows that list each neighbour once with the same coupling both ways).
+ * the next one's field; 6 every spin's local field in every slice of the
+ * swept parity kept on chip and updated on flips: up to 256 spins in the
+ * registers of a workgroup per replica, in blocks of 16 spins, else in LDS with
+ * one replica per wavefront (rows that list each neighbour once with the same
+ * coupling both ways).
  * 2-6 need rows that sum exactly in any order (piqmc_problem_exact_rows); a
  * sweep whose variant does not apply fails with PIQMC_EINVAL.  Every variant
  * gives identical results.  No reference counterpart. */
