@@ -2707,6 +2707,8 @@ size_t colored_scratch_bytes(const piqmc_problem *pb, int R, int P, int S)
     return b + CallBuffers::round_up(wb * 2 * (size_t)pb->N * R);
 }
 
+constexpr int kMaxRpw = 64;  // replicas a workgroup takes
+
 // Tile of the sparse real-coupling sweep (block 0: it does not apply).  The
 // caller's block and rpw are kept; by default a workgroup has the lanes that
 // take a slot's words (two color classes) in whole passes of at most 1024.
@@ -2715,7 +2717,7 @@ struct SparseTile {
 };
 SparseTile sparse_tile(const piqmc_problem *pb, int R, size_t word_bytes, int block, int rpw, bool chains)
 {
-    if (!pb->sparse_rows || block > 1024 || (block > 0 && (block & 63)) || rpw > 64) return {0, 0};
+    if (!pb->sparse_rows || block > 1024 || (block > 0 && (block & 63)) || rpw > kMaxRpw) return {0, 0};
     if (rpw <= 0) rpw = 1;
     if (block <= 0) {
         int most = 0;
@@ -2874,8 +2876,9 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         // the cached field sweep evaluates each step's decision classes once per
         // workgroup for all of its replicas: as many replicas per workgroup as
         // put every workgroup on the device at once (one 512-thread workgroup
-        // per CU), within the LDS (12^3 lattice with fields, P=128, 1024
-        // replicas, 100 sweeps: 4 per workgroup 8.3 ms, 2 9.6, 3 13.0, 1 12.0)
+        // per CU), within the LDS and the most a workgroup takes (12^3 lattice with
+        // fields, P=128, 1024 replicas, 100 sweeps: 4 per workgroup 8.3 ms, 2 9.6,
+        // 3 13.0, 1 12.0)
         int dev = 0, ncu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
@@ -2883,7 +2886,7 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         const size_t per = sizeof(WT) * 2 * (size_t)N;
         const size_t fixed_part = 4 * (kClassStride + 8) + 16 * sizeof(double) + (size_t)8 * kFieldCap * sizeof(uint2);
         const int lds_max = (int)std::max<size_t>(1, (160 * 1024 - fixed_part) / per);
-        rpw = std::max(1, std::min(lds_max, (R + ncu - 1) / ncu));
+        rpw = std::max(1, std::min(std::min(lds_max, kMaxRpw), (R + ncu - 1) / ncu));
     }
     if (rpw <= 0 && block <= 0 && fixed_tile_applies(pb, R, sizeof(WT))) {
         // the fixed-plane kernel's tile (1024-spin workload: 9.25 ms against
@@ -2892,7 +2895,7 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         block = (int)kFixBlock;
     }
     if (rpw <= 0) rpw = sparse ? tile.rpw : (R >= 2048 ? 4 : (R >= 1024 ? 2 : 1));
-    if (rpw > 64) return piqmc::set_error(PIQMC_EINVAL, "replicas per workgroup must be <= 64");
+    if (rpw > kMaxRpw) return piqmc::set_error(PIQMC_EINVAL, "replicas per workgroup must be <= 64");
     const size_t lds = sizeof(WT) * 2 * (size_t)N * rpw + 4 * (kClassStride + 8) + 16 * sizeof(double);
     if (lds > 160 * 1024)
         return piqmc::set_error(PIQMC_EINVAL, "colored sweep: replicas per workgroup x 2 x nspins x P/2 bits exceed one workgroup's LDS");

@@ -57,3 +57,38 @@ def test_open_bits_queue(gpu, L, dim, P, T, block, rpw):
                          trace=True)
         assert np.array_equal(c8[r].cpu().numpy(), ref)
         np.testing.assert_allclose(et[r].cpu().numpy(), e, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("L,dim,P", [(4, 2, 4), (8, 2, 66), (4, 3, 2)])
+def test_default_tile_of_many_replicas(gpu, L, dim, P):
+    """More replicas than 64 a compute unit, the most a workgroup takes, on
+    lattices of which more than 64 fit the LDS: default arguments run them."""
+    import torch
+    from piqmc import device
+    N, nbs, _, _, _ = pm_j_problem(L, dim=dim, seed=L + P, field_sigma=0.1)
+    R, S = 64 * torch.cuda.get_device_properties(0).multi_processor_count + 1, 2
+    sched = np.linspace(3.0, 1e-8, S)
+    pb = device.Problem(nbs)
+    color = pb.coloring()
+    g = torch.Generator(device=gpu).manual_seed(L)
+    c8 = torch.randint(0, 2, (R, P, N), generator=g, dtype=torch.int8, device=gpu) * 2 - 1
+    pick = (0, 63, 64, R // 2, R - 1)
+    init = {r: c8[r].cpu().numpy() for r in pick}
+    pb.qa_colored(c8, sched, 1, 1.0 / P, 5)
+    for r in pick:
+        O.qa_colored(sched, 1, P, 1.0 / P, init[r], nbs, color, int(color.max()) + 1, 5, replica=r)
+        assert np.array_equal(c8[r].cpu().numpy(), init[r])
+
+
+def test_default_tile_of_many_chains(gpu):
+    import torch
+    from piqmc import device
+    N, nbs, _, _, _ = pm_j_problem(4, seed=9, field_sigma=0.1)
+    pb = device.Problem(nbs)
+    # twice a prime: the chains are pairs, one replica each
+    C, sched = 2 * 20011, np.linspace(2.0, 0.1, 2)
+    s8 = torch.ones((C, N), dtype=torch.int8, device=gpu)
+    pb.sa_colored(s8, sched, 1, 7)
+    ref = np.ones((C, N), np.int8)
+    O.sa_colored(sched, 1, ref, nbs, pb.coloring(), pb.ncolors, 7)
+    assert np.array_equal(s8.cpu().numpy(), ref)
