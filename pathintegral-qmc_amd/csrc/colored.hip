@@ -2709,6 +2709,64 @@ size_t colored_scratch_bytes(const piqmc_problem *pb, int R, int P, int S)
 
 constexpr int kMaxRpw = 64;  // replicas a workgroup takes
 
+int biggest_class(const piqmc_problem *pb)
+{
+    int n = 0;
+    for (int c = 0; c < pb->ncolors; ++c) n = std::max(n, pb->color_off[c + 1] - pb->color_off[c]);
+    return n;
+}
+
+int cu_count()
+{
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
+        ncu = 256;
+    return ncu;
+}
+
+// The cached field sweep takes two colors of at most two spins per thread and
+// four or six couplings per spin besides the field (square and cubic
+// lattices): spins, neighbours and decision classes cached in registers.
+bool cached_fields_apply(const piqmc_problem *pb, int block)
+{
+    return pb->pmjf && !pb->pmj && pb->ncolors == 2 && (pb->zuni_nf == 4 || pb->zuni_nf == 6) && block <= 512 &&
+           biggest_class(pb) <= 2 * block && cached_fields_enabled();
+}
+size_t cached_fields_lds(int N, int rpw, int word_bytes, int block)
+{
+    return (size_t)word_bytes * 2 * N * rpw + 4 * (kClassStride + 8) + 16 * sizeof(double) +
+           (size_t)(block / 64) * kFieldCap * sizeof(uint2);
+}
+
+// Replicas per workgroup of the field sweep on square and cubic lattices.  A
+// workgroup evaluates a step's decision classes once for all of its replicas,
+// which costs about as much as sweeping two (8 x 8, P=20, 10 steps: 107 us
+// for one, 136, 171, 208 for two to four; 44 x 44 the same in its classes'
+// proportion).  A CU holds eight of the cached sweep's wavefronts (256
+// registers), so a call takes rounds = ceil(workgroups / what is resident) of
+// (2 + rpw) units, and the rpw of the fewest is taken.  8 x 8, P=128, 4096
+// replicas: 8 a workgroup 0.56 ms, 4 0.62, 16 1.01; 12^3, P=128, 1024: 4 8.3
+// ms (100 sweeps), 2 9.6, 3 13.0; 44 x 44, P=64, 4096: 8 1.90 ms, 9 2.09, 4
+// 2.15; 32 x 32, P=20, 8192: 8 1.63, 16 (one workgroup a CU) 2.29.  Larger
+// color classes leave the classes uncached; eight wavefronts a CU are what
+// pays there too (80 x 80, P=20, 1024 replicas: 2 1.32 ms, 3 1.65, 1 1.45).
+int fields_rpw(const piqmc_problem *pb, int R, int word_bytes, int block)
+{
+    const int ncu = cu_count();
+    const size_t queues = cached_fields_apply(pb, block) ? 0 : (size_t)(block / 64) * kFieldCap * sizeof(uint2);
+    int best = 1;
+    long long least = 0;
+    for (int rpw = 1; rpw <= std::min(R, kMaxRpw); ++rpw) {
+        const size_t lds = cached_fields_lds(pb->N, rpw, word_bytes, block) - queues;
+        if (lds > 160 * 1024) break;
+        const long long res = (long long)ncu * std::max(1, std::min((int)((160 * 1024) / lds), 512 / block));
+        const long long cost = (((R + rpw - 1) / rpw + res - 1) / res) * (2 + rpw);
+        if (rpw == 1 || cost < least) best = rpw, least = cost;
+    }
+    return best;
+}
+
 // Tile of the sparse real-coupling sweep (block 0: it does not apply).  The
 // caller's block and rpw are kept; by default a workgroup has the lanes that
 // take a slot's words (two color classes) in whole passes of at most 1024.
@@ -2870,24 +2928,8 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
     // per-bit general path
     const SparseTile tile = sparse_tile(pb, R, sizeof(WT), block, rpw, chains);
     const bool sparse = tile.block > 0;
-    const bool cached_fields = pb->pmjf && !pb->pmj && pb->ncolors == 2 && (pb->zuni_nf == 4 || pb->zuni_nf == 6) &&
-                               cached_fields_enabled();
-    if (rpw <= 0 && cached_fields) {
-        // the cached field sweep evaluates each step's decision classes once per
-        // workgroup for all of its replicas: as many replicas per workgroup as
-        // put every workgroup on the device at once (one 512-thread workgroup
-        // per CU), within the LDS and the most a workgroup takes (12^3 lattice with
-        // fields, P=128, 1024 replicas, 100 sweeps: 4 per workgroup 8.3 ms, 2 9.6,
-        // 3 13.0, 1 12.0)
-        int dev = 0, ncu = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1)
-            ncu = 256;
-        const size_t per = sizeof(WT) * 2 * (size_t)N;
-        const size_t fixed_part = 4 * (kClassStride + 8) + 16 * sizeof(double) + (size_t)8 * kFieldCap * sizeof(uint2);
-        const int lds_max = (int)std::max<size_t>(1, (160 * 1024 - fixed_part) / per);
-        rpw = std::max(1, std::min(std::min(lds_max, kMaxRpw), (R + ncu - 1) / ncu));
-    }
+    if (rpw <= 0 && pb->pmjf && !pb->pmj && pb->ncolors == 2 && (pb->zuni_nf == 4 || pb->zuni_nf == 6))
+        rpw = fields_rpw(pb, R, sizeof(WT), block > 0 ? block : (biggest_class(pb) > 512 ? 512 : 256));
     if (rpw <= 0 && block <= 0 && fixed_tile_applies(pb, R, sizeof(WT))) {
         // the fixed-plane kernel's tile (1024-spin workload: 9.25 ms against
         // 9.6 ms for the best general tile)
@@ -2904,8 +2946,7 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         // 256 threads; 512 when a color class would take more than two passes
         // of 256 (measured on the 1728-spin 3-D lattice: 1.08e12 vs 0.84e12
         // attempts/s)
-        int biggest = 0;
-        for (int c = 0; c < pb->ncolors; ++c) biggest = std::max(biggest, pb->color_off[c + 1] - pb->color_off[c]);
+        const int biggest = biggest_class(pb);
         block = biggest > 512 ? 512 : 256;
         if (pmj && pb->zuni >= 0) {
             if (pb->ncolors == 2) {
@@ -2959,13 +3000,8 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         if ((rc = piqmc::sparse_launch(c, st))) return rc;
     } else if (!pmj && pb->pmjf) {
         a.zuni = -1;
-        int biggest = 0;
-        for (int c = 0; c < pb->ncolors; ++c) biggest = std::max(biggest, pb->color_off[c + 1] - pb->color_off[c]);
-        // two colors of at most two spins per thread and four or six couplings
-        // per spin besides the field (square and cubic lattices): spins,
-        // neighbours and decision classes cached in registers
-        const size_t lf = lds + (size_t)(block / 64) * kFieldCap * sizeof(uint2);
-        if (biggest <= 2 * block && block <= 512 && lf <= 160 * 1024 && cached_fields) {
+        const size_t lf = cached_fields_lds(N, rpw, sizeof(WT), block);
+        if (cached_fields_apply(pb, block) && lf <= 160 * 1024) {
             auto kern = pb->zuni_nf == 4 ? colored_fields_cached_kernel<WT, 4> : colored_fields_cached_kernel<WT, 6>;
             (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lf);
             kern<<<grid, block, lf, st>>>(a);

@@ -92,3 +92,27 @@ def test_default_tile_of_many_chains(gpu):
     ref = np.ones((C, N), np.int8)
     O.sa_colored(sched, 1, ref, nbs, pb.coloring(), pb.ncolors, 7)
     assert np.array_equal(s8.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("L,dim,P,R", [(8, 2, 128, 4096), (80, 2, 20, 1024), (12, 3, 20, 4096), (8, 3, 64, 2100)])
+def test_default_tile_is_near_the_best(gpu, L, dim, P, R):
+    """The kernel time of the default replicas per workgroup against that of every
+    smaller power of two and their multiples of three."""
+    import torch
+    from piqmc import device
+    N, nbs, _, _, _ = pm_j_problem(L, dim=dim, seed=L + P, field_sigma=0.1)
+    pb = device.Problem(nbs)
+    c8 = torch.ones((R, P, N), dtype=torch.int8, device=gpu)
+    sched = np.linspace(3.0, 1e-8, 6)
+
+    def ms(rpw):
+        best = np.inf
+        for _ in range(5):
+            c8.fill_(1)
+            pb.qa_colored(c8, sched, 1, 1.0 / P, 5, rpw=rpw)
+            best = min(best, device.last_kernel_ms())
+        return best
+
+    word = 4 if P <= 64 else 8
+    fits = [r for r in (1, 2, 3, 4, 6, 8, 12, 16) if 2 * N * word * r < 150000]
+    assert ms(0) <= 1.2 * min(ms(r) for r in fits)
