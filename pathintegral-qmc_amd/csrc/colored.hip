@@ -21,6 +21,7 @@
 // decisions of piqmc_fixed_class with the draw
 //   philox(key=seed, ctr={sweep, spin, replica, tau<<24 | m>>2})[m&3]
 // for bit m, so the result does not depend on workgroup size or scheduling.
+#include <limits.h>
 #include <math.h>
 
 #include <algorithm>
@@ -2767,6 +2768,46 @@ int fields_rpw(const piqmc_problem *pb, int R, int word_bytes, int block)
     return best;
 }
 
+// Threads per workgroup of the word-per-thread sweep.
+int default_block(const piqmc_problem *pb, int R, int rpw, int word_bytes, bool pmj)
+{
+    // 256 threads; 512 when a color class would take more than two passes
+    // of 256 (measured on the 1728-spin 3-D lattice: 1.08e12 vs 0.84e12
+    // attempts/s)
+    const int biggest = biggest_class(pb), block = biggest > 512 ? 512 : 256;
+    if (!pmj || pb->zuni < 0) return block;
+    if (pb->ncolors == 2) {
+        // 1024 where that keeps two spins a thread, so that neighbours stay
+        // in registers (64 x 64, P=40: 4 replicas, 40 steps 589 -> 406 us; 512
+        // replicas, 20 steps 498 -> 454), and the queues still fit
+        if (biggest > 1024 && biggest <= 2048 && queue_lds(pb->N, rpw, word_bytes, 1024) <= 160 * 1024) return 1024;
+        return block;
+    }
+    // More colors reload their neighbours, and nothing but a class's passes asks
+    // for threads.  512 have the fewer passes; 256 where they bring the call's
+    // workgroups onto the device in fewer rounds, of 16 wavefronts a CU (more
+    // gain nothing) within the LDS, or where the classes are so small that the
+    // draws' partial batches, with which every wavefront ends a phase, weigh
+    // more.  10 steps, 256 / 512 threads in us: 55 x 55, P=20: 301 replicas 212
+    // / 184, 600 246 / 288, 1000 285 / 348; 65 x 65, P=128, 600: 1011 / 755; 99
+    // x 99, P=20, 300: 884 / 579; 17^3, P=20, 600: 549 / 423; 33 x 33, P=50,
+    // 301 (100 steps): 1107 / 1157, and 41 x 41: 1452 / 1324.
+    const int ncu = cu_count(), G = (R + rpw - 1) / rpw;
+    const bool queued = word_bytes == 4 && queue_enabled();
+    auto rounds = [&](int threads) -> int {
+        constexpr size_t kUnit = 1280;  // LDS is allocated in these
+        const size_t lds = (queued ? queue_lds(pb->N, rpw, word_bytes, threads) : queue_offset(pb->N, rpw, word_bytes)) +
+                           kUnit - 1;
+        if (lds / kUnit * kUnit > 160 * 1024) return INT_MAX;  // (then without the queues)
+        const int res = ncu * std::min((int)(160 * 1024 / (lds / kUnit * kUnit)), 1024 / threads);
+        return (G + res - 1) / res;
+    };
+    if (biggest <= 256) return 256;
+    const int r256 = rounds(256), r512 = rounds(512);
+    if (r256 != r512) return r256 < r512 ? 256 : 512;
+    return queued && G > ncu && rpw * biggest <= 640 ? 256 : 512;
+}
+
 // Tile of the sparse real-coupling sweep (block 0: it does not apply).  The
 // caller's block and rpw are kept; by default a workgroup has the lanes that
 // take a slot's words (two color classes) in whole passes of at most 1024.
@@ -2942,29 +2983,7 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
     if (lds > 160 * 1024)
         return piqmc::set_error(PIQMC_EINVAL, "colored sweep: replicas per workgroup x 2 x nspins x P/2 bits exceed one workgroup's LDS");
     if (block <= 0 && sparse) block = tile.block;
-    if (block <= 0) {
-        // 256 threads; 512 when a color class would take more than two passes
-        // of 256 (measured on the 1728-spin 3-D lattice: 1.08e12 vs 0.84e12
-        // attempts/s)
-        const int biggest = biggest_class(pb);
-        block = biggest > 512 ? 512 : 256;
-        if (pmj && pb->zuni >= 0) {
-            if (pb->ncolors == 2) {
-                // 1024 where that keeps two spins a thread, so that neighbours stay
-                // in registers (64 x 64, P=40: 4 replicas, 40 steps 589 -> 406 us; 512
-                // replicas, 20 steps 498 -> 454), and the queues still fit
-                if (biggest > 1024 && biggest <= 2048 && queue_lds(N, rpw, sizeof(WT), 1024) <= 160 * 1024) block = 1024;
-            } else {
-                // more colors reload their neighbours: with a workgroup a CU, 512
-                // threads for the latency of a class's passes (25 x 25, P=100, 200
-                // replicas 739 -> 643 us; 9^3, P=64, 100 replicas 474 -> 432); with
-                // several, 256 for the draws' partial batches a wavefront ends
-                // each phase with (33 x 33, P=50: 301 replicas 1655 -> 1572 us, 2000
-                // 1435 -> 1264; 11^3, P=64, 800 replicas 757 -> 664)
-                block = biggest > 256 && (R + rpw - 1) / rpw <= 256 ? 512 : 256;
-            }
-        }
-    }
+    if (block <= 0) block = default_block(pb, R, rpw, sizeof(WT), pmj);
     if (block > 1024 || (block & 63)) return piqmc::set_error(PIQMC_EINVAL, "block must be a multiple of 64, <= 1024");
     float *d_jp = nullptr;  // [S] J_perp, then [S] temperatures
     uint32_t *d_thr = nullptr, *d_zt = nullptr;

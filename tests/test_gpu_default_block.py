@@ -28,3 +28,30 @@ def test_default_block(gpu, L, dim, P, R):
         ref = init[r].copy()
         O.qa_colored(sched, 1, P, T, ref, nbs, color, int(color.max()) + 1, 5, replica=r)
         assert np.array_equal(c8[r].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("L,dim,P,R", [(99, 2, 20, 300), (65, 2, 128, 600), (17, 3, 20, 600), (25, 2, 64, 1000),
+                                       (33, 2, 100, 301), (33, 2, 20, 2048)])
+def test_default_block_is_near_the_best(gpu, L, dim, P, R):
+    """More than two colors: the kernel time of the default workgroup size against
+    that of 256 and of 512 threads."""
+    _near_the_best(gpu, L, dim, P, R, (256, 512))
+
+
+def _near_the_best(gpu, L, dim, P, R, blocks):
+    import torch
+    from piqmc import device
+    N, nbs, _, _, _ = pm_j_problem(L, dim=dim, seed=L + P)
+    pb = device.Problem(nbs)
+    c8 = torch.ones((R, P, N), dtype=torch.int8, device=gpu)
+    sched = np.linspace(3.0, 1e-8, 20)
+
+    def ms(block):
+        best = np.inf
+        for _ in range(6):
+            c8.fill_(1)
+            pb.qa_colored(c8, sched, 1, 1.0 / P, 5, block=block)
+            best = min(best, device.last_kernel_ms())
+        return best
+
+    assert ms(0) <= 1.1 * min(ms(b) for b in blocks)
