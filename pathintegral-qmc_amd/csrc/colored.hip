@@ -2777,10 +2777,17 @@ int default_block(const piqmc_problem *pb, int R, int rpw, int word_bytes, bool 
     const int biggest = biggest_class(pb), block = biggest > 512 ? 512 : 256;
     if (!pmj || pb->zuni < 0) return block;
     if (pb->ncolors == 2) {
-        // 1024 where that keeps two spins a thread, so that neighbours stay
-        // in registers (64 x 64, P=40: 4 replicas, 40 steps 589 -> 406 us; 512
-        // replicas, 20 steps 498 -> 454), and the queues still fit
-        if (biggest > 1024 && biggest <= 2048 && queue_lds(pb->N, rpw, word_bytes, 1024) <= 160 * 1024) return 1024;
+        // 1024 where that keeps two spins a thread, so that neighbours stay in
+        // registers (64 x 64, P=40: 4 replicas, 40 steps 589 -> 406 us; 512 replicas,
+        // 20 steps 498 -> 454), and the queues still fit.  Two 512-thread workgroups
+        // a CU do better on words of 32 bits while a replica or two leave many of
+        // those threads without a second spin (46 x 46, 1058 spins a color, P=20:
+        // 600 replicas 170 us at 512, 208 at 1024; 14^3, 1372, P=64, 600: 208 / 237; 56
+        // x 56, 1568, P=20, 600: 244 / 227; 46 x 46, 2048 replicas, four a workgroup:
+        // 384 / 295; 10 steps each); with a workgroup a CU its time is all that counts.
+        const bool filled = word_bytes == 8 || biggest > 1536 || rpw >= 4 || (R + rpw - 1) / rpw <= cu_count();
+        if (biggest > 1024 && biggest <= 2048 && filled && queue_lds(pb->N, rpw, word_bytes, 1024) <= 160 * 1024)
+            return 1024;
         return block;
     }
     // More colors reload their neighbours, and nothing but a class's passes asks

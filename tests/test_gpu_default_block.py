@@ -55,3 +55,9 @@ def _near_the_best(gpu, L, dim, P, R, blocks):
         return best
 
     assert ms(0) <= 1.1 * min(ms(b) for b in blocks)
+
+
+@pytest.mark.parametrize("L,dim,P,R", [(46, 2, 20, 600), (14, 3, 20, 1000), (46, 2, 64, 100), (46, 2, 128, 600),
+                                       (64, 2, 64, 600), (46, 2, 20, 2048)])
+def test_default_block_of_two_large_colors(gpu, L, dim, P, R):
+    _near_the_best(gpu, L, dim, P, R, (512, 1024))
