@@ -2675,7 +2675,8 @@ int upload_tables(CallBuffers &buf, std::initializer_list<Table> tables)
     size_t total = 0;
     for (const Table &t : tables) total += CallBuffers::round_up(t.bytes);
     unsigned char *base = nullptr;
-    int rc = buf.take((void **)&base, total);
+    // (a call without field steps may have none: a byte's room, nothing to copy)
+    int rc = buf.take((void **)&base, total ? total : 1);
     if (rc) return rc;
     std::vector<unsigned char> host(total);
     size_t at = 0;
@@ -2684,7 +2685,7 @@ int upload_tables(CallBuffers &buf, std::initializer_list<Table> tables)
         *t.dst = base + at;
         at += CallBuffers::round_up(t.bytes);
     }
-    PIQMC_HIP(hipMemcpyAsync(base, host.data(), total, hipMemcpyHostToDevice, buf.st));
+    if (total) PIQMC_HIP(hipMemcpyAsync(base, host.data(), total, hipMemcpyHostToDevice, buf.st));
     return PIQMC_OK;
 }
 

@@ -61,3 +61,29 @@ def test_blocked_chains_match_oracle(gpu, N, C):
     pb.sa_colored(d, sched, 2, seed=5)
     O.sa_colored(sched, 2, ref, nbs, pb.coloring(), pb.ncolors, 5)
     assert np.array_equal(d.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("variant", ["auto", "wave", "split", "workgroup", "pipe4", "fields"])
+def test_no_field_steps(gpu, variant):
+    """A call without field steps is the identity on every dense layout, with
+    and without a scratch region, and leaves no error for the call after it."""
+    import ctypes as C
+    import torch
+    from piqmc import _lib, device
+    rng = np.random.RandomState(1)
+    nbs = _dense(48, rng)
+    pb = device.Problem(nbs)
+    pb.set_dense_variant(variant)
+    init = (2 * rng.randint(2, size=(3, 16, 48)) - 1).astype(np.int8)
+    d = torch.from_numpy(init.copy()).to(gpu)
+    none = np.zeros(0)
+    for _ in range(2):
+        assert pb.qa_colored(d, none, 1, 0.1, 1, trace=True).shape == (3, 0)
+        _lib.call("piqmc_qa_colored_noalloc", pb._h, 3, 16, 0, 1, 0.1, none.ctypes.data, d.data_ptr(), 1, 0, 0, None,
+                  0, 0, C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert np.array_equal(d.cpu().numpy(), init)
+    sched = np.linspace(3.0, 1e-8, 4)
+    pb.qa_colored(d, sched, 1, 1 / 16, 7)
+    ref = init[0].copy()
+    O.qa_colored(sched, 1, 16, 1 / 16, ref, nbs, pb.coloring(), pb.ncolors, 7)
+    assert np.array_equal(d[0].cpu().numpy(), ref)
