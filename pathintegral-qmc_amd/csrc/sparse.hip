@@ -302,8 +302,12 @@ __global__ void __launch_bounds__(1024) sparse_kernel(SparseArgs<WT> a)
                 uint32_t aw[places<ZK> / 4];
                 __builtin_memcpy(aw, __builtin_assume_aligned(a.t.w + (size_t)q * (places<ZK> / 4), places<ZK>),
                                  places<ZK>);
-                // thresholds on the count, per u_t: accept from ka, reject
-                // below kr; `fin` false (T <= 0, infinite J_perp) leaves all open
+                // thresholds on the count, per u_t: accept from pa, reject
+                // below pr; T <= 0 or an infinite J_perp leaves all open.  A product
+                // v or w past float's range makes the sums infinite, which leaves the
+                // attempt open, or inf - inf, which the clamp makes 0: open below, and
+                // accepted at two antiparallel Trotter bonds, where 4 J_perp is then
+                // 1e36 times what the row could hold against it.
                 uint32_t pa = 0x00ffffffu, pr = 0;
                 if (T > 0.0f && T < INFINITY && fabsf(jp) < INFINITY) {
                     const float c = __uint_as_float(mt.y), v = c * jp, w = 5.875f * c * T;

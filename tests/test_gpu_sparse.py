@@ -71,3 +71,23 @@ def test_sparse_chains_match_oracle(gpu, kind, C):
     pb.sa_colored(d, sched, 2, seed=31, replica_base=2, sweep_base=1)
     O.sa_colored(sched, 2, ref, nbs, pb.coloring(), pb.ncolors, 31, replica_base=2, sweep_base=1)
     assert np.array_equal(d.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("scale,T", [(1e-28, 1e9), (1e-28, 1.0), (1e-20, 1e20), (1e20, 1e-3), (1e27, 1e9)])
+def test_scales_past_float_products(gpu, scale, T):
+    """Couplings and temperatures of which a product (weight scale times J_perp or
+    T) leaves float's range: the filter then decides nothing wrongly."""
+    import torch
+    from piqmc import device, instances
+    rng = np.random.RandomState(3)
+    N, r, c, v = instances.lattice_pm_j(6, 2, rng, 0.0)
+    nbs = instances.neighbors(N, r, c, scale * rng.randn(v.size))
+    pb = device.Problem(nbs)
+    P, R, sched = 20, 3, np.array([3.0, 1.0, 1e-3, 1e-8])
+    init = (2 * rng.randint(2, size=(R, P, N)) - 1).astype(np.int8)
+    d = torch.from_numpy(init.copy()).to(gpu)
+    pb.qa_colored(d, sched, 2, T, 9)
+    for k in range(R):
+        ref = init[k].copy()
+        O.qa_colored(sched, 2, P, T, ref, nbs, pb.coloring(), pb.ncolors, 9, replica=k)
+        assert np.array_equal(d[k].cpu().numpy(), ref)
