@@ -1330,6 +1330,16 @@ inline bool dense_wg_enabled()
     return !(e && e[0] == '0');
 }
 
+// Whether the blocked dense sweep runs problem pb in a layout that leaves the
+// choice (automatic, or cached fields).  The switches that compare the other
+// dense layouts choose among those: with any of them set it stands back.
+inline bool block_sweep_runs(const piqmc_problem *pb)
+{
+    for (const char *s : {"PIQMC_DENSE_WG", "PIQMC_DENSE_PIPE", "PIQMC_DENSE_PIPE_WAVES", "PIQMC_FIELDS_SPLIT"})
+        if (std::getenv(s)) return false;
+    return piqmc::block_applies(pb);
+}
+
 // The cached-register field sweep (PIQMC_CACHED_FIELDS=0 selects the general
 // one, for comparisons).
 inline bool cached_fields_enabled()
@@ -2867,7 +2877,7 @@ int run_colored(const piqmc_problem *pb, int R, int P, int S, int M,
         int pw = 4;
         size_t lwg = 0;
         bool fields_auto = false;
-        const bool block_sweep = (pb->dense_variant == 0 || pb->dense_variant == 6) && piqmc::block_applies(pb);
+        const bool block_sweep = (pb->dense_variant == 0 || pb->dense_variant == 6) && block_sweep_runs(pb);
         if (block_sweep) {
             // blocks of spins, both parities at once (dense_block.hip): faster at
             // every slice and replica count measured (2 to 8192 replicas)

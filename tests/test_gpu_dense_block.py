@@ -87,3 +87,36 @@ def test_no_field_steps(gpu, variant):
     ref = init[0].copy()
     O.qa_colored(sched, 1, 16, 1 / 16, ref, nbs, pb.coloring(), pb.ncolors, 7)
     assert np.array_equal(d[0].cpu().numpy(), ref)
+
+
+SWITCHES = ("PIQMC_DENSE_WG", "PIQMC_DENSE_PIPE", "PIQMC_DENSE_PIPE_WAVES", "PIQMC_FIELDS_SPLIT")
+
+
+@pytest.mark.parametrize("P,switch,value,items", [
+    (16, None, "", 8), (66, None, "", 8), (16, "PIQMC_DENSE_WG", "0", 2), (66, "PIQMC_DENSE_WG", "0", 2),
+    (16, "PIQMC_FIELDS_SPLIT", "0", 2), (66, "PIQMC_FIELDS_SPLIT", "0", 2), (66, "PIQMC_FIELDS_SPLIT", "1", 2),
+    (16, "PIQMC_FIELDS_SPLIT", "1", 8)])
+def test_layout_switches_reach_a_batch(gpu, monkeypatch, P, switch, value, items):
+    """A replica per work item in the blocked sweep, four in the layouts that the
+    switches compare (one where the replica's 8 slices a parity are split over the
+    four wavefronts; 33 are not); the same spins from all of them."""
+    import torch
+    from piqmc import device
+    for s in SWITCHES:
+        monkeypatch.delenv(s, raising=False)
+    if switch:
+        monkeypatch.setenv(switch, value)
+    rng = np.random.RandomState(2)
+    nbs = _dense(24, rng)
+    pb = device.Problem(nbs)
+    init = (2 * rng.randint(2, size=(8, P, 24)) - 1).astype(np.int8)
+    d = torch.from_numpy(init.copy()).to(gpu)
+    sched = np.linspace(3.0, 1e-8, 5)
+    b = device.Batch()
+    b.add(pb, d, sched, 1, 1.0 / P, 7)
+    b.run()
+    assert b.info()["items"] == items
+    for r in range(8):
+        ref = init[r].copy()
+        O.qa_colored(sched, 1, P, 1.0 / P, ref, nbs, pb.coloring(), pb.ncolors, 7, replica=r)
+        assert np.array_equal(d[r].cpu().numpy(), ref)
