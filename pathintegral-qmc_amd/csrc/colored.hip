@@ -2702,12 +2702,13 @@ int upload_tables(CallBuffers &buf, std::initializer_list<Table> tables)
 // Device bytes a parallel-sweep call takes from a CallBuffers region (each
 // buffer rounded up to 256 bytes): J_perp and temperatures [2S] floats, the
 // +-1 path's per-step tables, the color offsets and the packed state
-// [R][2][N] words.
+// [R][2][N] words; the local fields where the cached-field dense sweep may
+// run (the blocked one keeps them on chip).
 size_t colored_scratch_bytes(const piqmc_problem *pb, int R, int P, int S)
 {
     const size_t wb = P / 2 <= 32 ? 4 : 8;
     size_t b = CallBuffers::round_up(sizeof(float) * (S ? 2 * S : 1));
-    if (use_dense(pb) && pb->Z <= kFieldsMaxRow &&
+    if (use_dense(pb) && pb->Z <= kFieldsMaxRow && !block_sweep_runs(pb) &&
         (pb->dense_variant == 6 || (pb->dense_variant == 0 && pb->exact_rows && pb->fields_ok)))
         b += CallBuffers::round_up(sizeof(double) * 2 * (size_t)(P / 2) * (pb->N | 1) * R);
     if (!use_dense(pb)) {

@@ -120,3 +120,33 @@ def test_layout_switches_reach_a_batch(gpu, monkeypatch, P, switch, value, items
         ref = init[r].copy()
         O.qa_colored(sched, 1, P, 1.0 / P, ref, nbs, pb.coloring(), pb.ncolors, 7, replica=r)
         assert np.array_equal(d[r].cpu().numpy(), ref)
+
+
+def test_scratch_counts_what_the_blocked_sweep_takes(gpu, monkeypatch):
+    """The region of the allocation-free entry holds 300 replicas of 256 spins at
+    P=128 (4 KiB each); cached fields, 257 KiB a replica more, would not fit it."""
+    import ctypes as C
+    import torch
+    from piqmc import _lib, device
+    for s in SWITCHES:
+        monkeypatch.delenv(s, raising=False)
+    rng = np.random.RandomState(5)
+    pb = device.Problem(_dense(256, rng))
+    P, sched = 128, np.linspace(3.0, 1e-8, 2)
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def noalloc(d, R):
+        _lib.call("piqmc_qa_colored_noalloc", pb._h, R, P, 2, 1, 1.0 / P, sched.ctypes.data, d.data_ptr(), 9, 0, 0, None,
+                  0, 0, st)
+
+    a = torch.from_numpy((2 * rng.randint(2, size=(300, P, 256)) - 1).astype(np.int8)).to(gpu)
+    b = a.clone()
+    noalloc(a, 300)
+    pb.qa_colored(b, sched, 1, 1.0 / P, 9)
+    assert torch.equal(a, b)
+    need = 20000 * 8 * 2 * 256 + 256      # refused before any device work
+    with pytest.raises(ValueError, match=" %d bytes" % need):
+        noalloc(a, 20000)
+    monkeypatch.setenv("PIQMC_FIELDS_SPLIT", "0")
+    with pytest.raises(ValueError, match=" %d bytes" % (need + 20000 * 8 * 2 * 64 * 257)):
+        noalloc(a, 20000)
