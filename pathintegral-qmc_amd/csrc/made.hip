@@ -889,45 +889,74 @@ __global__ void sample_step(const float *logits, int B, int N, int d, const uint
 namespace {
 int up64(int n) { return (n + 63) & ~63; }
 
-// Row pitches of the layers' inputs and of the logits (multiples of 64; what
-// lies past the sizes is zeroed here and never written).
+int grid1(size_t n) { return (int)std::min<size_t>((n + 255) / 256, 65535); }
+
+// Columns [cols, pitch) of rows [0, rows) to zero.
+__global__ void zero_pad(uint16_t *p, size_t rows, int cols, int pitch)
+{
+    const int w = pitch - cols;
+    for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < rows * w; t += (size_t)gridDim.x * blockDim.x)
+        p[t / w * pitch + cols + t % w] = 0;
+}
+
+// The buffers of a forward pass over B rows.  Row pitches of the layers' inputs
+// are multiples of 64; nothing of a forward pass reads or writes past the sizes.
 int made_alloc_batch(piqmc_made *m, int B)
 {
     if (B <= m->cap) return PIQMC_OK;
-    const int N = m->N, H1 = m->H1, H2 = m->H2, lN = up64(N), l1 = up64(H1), l2 = up64(H2), lB = up64(B);
-    void **bufs[] = {(void **)&m->x, (void **)&m->h1, (void **)&m->h2, (void **)&m->logits, (void **)&m->dlog,
-                     (void **)&m->dh2, (void **)&m->dh1, (void **)&m->xt, (void **)&m->h1t, (void **)&m->h2t,
-                     (void **)&m->dlogt, (void **)&m->dh2t, (void **)&m->dh1t, (void **)&m->nll, (void **)&m->s};
+    void **bufs[] = {(void **)&m->x, (void **)&m->h1, (void **)&m->h2, (void **)&m->logits, (void **)&m->nll,
+                     (void **)&m->s};
     for (auto p : bufs)
         if (*p) (void)hipFree(*p), *p = nullptr;
     m->cap = 0;
+    m->padded = 0;
     if (m->gexec) (void)hipGraphExecDestroy(m->gexec), m->gexec = nullptr, m->gB = 0;  // holds old addresses
-    auto zeroed = [](uint16_t **p, size_t n) -> hipError_t {
-        hipError_t e = hipMalloc((void **)p, 2 * n);
-        return e == hipSuccess ? hipMemset(*p, 0, 2 * n) : e;
-    };
-    PIQMC_HIP(zeroed(&m->x, (size_t)B * lN));
-    PIQMC_HIP(zeroed(&m->h1, (size_t)B * l1));
-    PIQMC_HIP(zeroed(&m->h2, (size_t)B * l2));
-    PIQMC_HIP(hipMalloc(&m->logits, 4 * (size_t)B * N));
-    PIQMC_HIP(zeroed(&m->dlog, (size_t)B * lN));
-    PIQMC_HIP(zeroed(&m->dh2, (size_t)B * l2));
-    PIQMC_HIP(zeroed(&m->dh1, (size_t)B * l1));
-    PIQMC_HIP(zeroed(&m->xt, (size_t)N * lB));
-    PIQMC_HIP(zeroed(&m->h1t, (size_t)H1 * lB));
-    PIQMC_HIP(zeroed(&m->h2t, (size_t)H2 * lB));
-    PIQMC_HIP(zeroed(&m->dlogt, (size_t)N * lB));
-    PIQMC_HIP(zeroed(&m->dh2t, (size_t)H2 * lB));
-    PIQMC_HIP(zeroed(&m->dh1t, (size_t)H1 * lB));
+    PIQMC_HIP(hipMalloc(&m->x, 2 * (size_t)B * up64(m->N)));
+    PIQMC_HIP(hipMalloc(&m->h1, 2 * (size_t)B * up64(m->H1)));
+    PIQMC_HIP(hipMalloc(&m->h2, 2 * (size_t)B * up64(m->H2)));
+    PIQMC_HIP(hipMalloc(&m->logits, 4 * (size_t)B * m->N));
     PIQMC_HIP(hipMalloc(&m->nll, 8 * (size_t)B));
-    PIQMC_HIP(hipMalloc(&m->s, (size_t)B * N));
-    // the zeroing runs on the null stream, the callers' streams need not wait for it
-    PIQMC_HIP(hipDeviceSynchronize());
+    PIQMC_HIP(hipMalloc(&m->s, (size_t)B * m->N));
     m->cap = B;
     return PIQMC_OK;
 }
 
-int grid1(size_t n) { return (int)std::min<size_t>((n + 255) / 256, 65535); }
+// Those and the buffers of a training step, of a capacity of their own, so that
+// drawing and scoring slices does not pay for them.  The fused products read
+// whole stages of 64 columns: what lies past the sizes is zeroed here, on the
+// step's stream, and never written.  (The transposed buffers are written in
+// whole tiles by every step.)
+int made_alloc_train(piqmc_made *m, int B, hipStream_t st)
+{
+    if (const int rc = made_alloc_batch(m, B)) return rc;
+    const int N = m->N, H1 = m->H1, H2 = m->H2, lN = up64(N), l1 = up64(H1), l2 = up64(H2);
+    if (B > m->tcap) {
+        const size_t lB = up64(B);
+        void **bufs[] = {(void **)&m->dlog, (void **)&m->dh2, (void **)&m->dh1, (void **)&m->xt, (void **)&m->h1t,
+                         (void **)&m->h2t, (void **)&m->dlogt, (void **)&m->dh2t, (void **)&m->dh1t};
+        const size_t n[] = {(size_t)B * lN, (size_t)B * l2, (size_t)B * l1, N * lB, H1 * lB, H2 * lB, N * lB, H2 * lB, H1 * lB};
+        for (auto p : bufs)
+            if (*p) (void)hipFree(*p), *p = nullptr;
+        m->tcap = 0;
+        m->padded = 0;
+        for (int k = 0; k < 9; ++k) PIQMC_HIP(hipMalloc(bufs[k], 2 * n[k]));
+        m->tcap = B;
+    }
+    if (!m->padded) {
+        auto pad = [&](uint16_t *p, int rows, int cols) {
+            if (cols % 64) zero_pad<<<grid1((size_t)rows * (up64(cols) - cols)), 256, 0, st>>>(p, rows, cols, up64(cols));
+        };
+        pad(m->x, m->cap, N);
+        pad(m->h1, m->cap, H1);
+        pad(m->h2, m->cap, H2);
+        pad(m->dlog, m->tcap, N);
+        pad(m->dh2, m->tcap, H2);
+        pad(m->dh1, m->tcap, H1);
+        PIQMC_HIP(hipGetLastError());
+        m->padded = 1;
+    }
+    return PIQMC_OK;
+}
 
 void transpose(const uint16_t *in, int R, int C, int ldi, uint16_t *out, int ldo, hipStream_t st)
 {
@@ -1105,7 +1134,7 @@ int train_core(piqmc_made *m, int B, const int8_t *s, const int32_t *perm, int b
                hipStream_t st)
 {
     const int N = m->N, H1 = m->H1, H2 = m->H2;
-    const int lN = up64(N), l1 = up64(H1), l2 = up64(H2), lB = up64(m->cap);
+    const int lN = up64(N), l1 = up64(H1), l2 = up64(H2), lB = up64(m->tcap);
     const int kf[3] = {train_groups(B, H1, N), train_groups(B, H2, H1), train_groups(B, N, H2)};
     const int kd[2] = {train_groups(B, H1, H2), train_groups(B, H2, N)};  // dh1, dh2
     const int kw[3] = {train_groups(H1, N, B), train_groups(H2, H1, B), train_groups(N, H2, B)};
@@ -1222,9 +1251,9 @@ extern "C" int piqmc_made_train_step(piqmc_made *m, int B, const int8_t *s_dev, 
                                      void *stream)
 {
     if (!m || B < 1 || !s_dev) return piqmc::set_error(PIQMC_EINVAL, "made_train_step: bad args");
-    int rc = made_alloc_batch(m, B);
-    if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
+    int rc = made_alloc_train(m, B, st);
+    if (rc) return rc;
     rc = train_core(m, B, s_dev, nullptr, 0, lr, m->nll, st);
     if (rc) return rc;
     if (mean_nll) {
@@ -1246,9 +1275,9 @@ extern "C" int piqmc_made_train_epoch(piqmc_made *m, int n, const int8_t *data_d
 {
     if (!m || n < 1 || batch < 1 || batch > n || !data_dev || !perm_dev)
         return piqmc::set_error(PIQMC_EINVAL, "made_train_epoch: bad args");
-    int rc = made_alloc_batch(m, batch);
-    if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
+    int rc = made_alloc_train(m, batch, st);
+    if (rc) return rc;
     const int steps = n / batch;
     // per-row NLL of every step, then the steps' sums
     const size_t need = (size_t)steps * batch + steps;

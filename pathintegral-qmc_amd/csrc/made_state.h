@@ -6,17 +6,18 @@
 
 // ------------------------------------------------------------------ MADE state
 struct piqmc_made {
-    int N = 0, H1 = 0, H2 = 0, cap = 0;  // cap = max batch rows of the buffers
+    int N = 0, H1 = 0, H2 = 0, cap = 0, tcap = 0;  // most batch rows of the forward buffers, of the training ones
+    int padded = 0;  // what lies past the sizes in their rows is zero
     int layers_in[3], layers_out[3];
     float *w[3] = {}, *b[3] = {}, *mw[3] = {}, *vw[3] = {}, *mb[3] = {}, *vb[3] = {};
     uint16_t *wb[3] = {}, *wt[3] = {};   // bf16 [out][in], [in][out], row pitches rounded up to 64, zeros past the sizes
     uint8_t *mask[3] = {};
     float *gw[3] = {}, *gb[3] = {};
-    // activations [cap][*], row pitches (but the logits') rounded up to 64, zeros past the sizes
+    // activations [cap][*] and their gradients [tcap][*], row pitches (but the logits') rounded up to 64
     uint16_t *x = nullptr, *h1 = nullptr, *h2 = nullptr;
     float *logits = nullptr;
     uint16_t *dlog = nullptr, *dh2 = nullptr, *dh1 = nullptr;
-    // transposes for the weight gradients [units][cap rounded up to 64]
+    // transposes for the weight gradients [units][tcap rounded up to 64]
     uint16_t *xt = nullptr, *h1t = nullptr, *h2t = nullptr, *dlogt = nullptr, *dh2t = nullptr, *dh1t = nullptr;
     double *nll = nullptr;
     int8_t *s = nullptr;
