@@ -519,7 +519,7 @@ __global__ void spins_to_bf16(const int8_t *s, int B, int N, uint16_t *x, int ld
 {
     const size_t n = (size_t)B * N;
     for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x)
-        x[t / N * ldx + t % N] = s[t] < 0 ? 0xBF80u : 0x3F80u;  // -1.0 / +1.0 in bf16
+        x[ldx == N ? t : t / N * ldx + t % N] = s[t] < 0 ? 0xBF80u : 0x3F80u;  // -1.0 / +1.0 in bf16
 }
 
 // transpose bf16 [R][ldi] -> [C][ldo]
