@@ -15,13 +15,18 @@ The sweep's tiles change only speed: every choice takes identical decisions
 ``tune_colored`` times each candidate on a short schedule that samples the
 real one (the cost per attempt depends on the field: how many bits need a
 random draw), keeps the fastest, and caches it in a JSON file keyed by device
-architecture and problem shape; ``tune_batch`` does the same for a batch on
+architecture, library build and problem shape (a tile timed on other kernels
+says nothing about these); ``tune_batch`` does the same for a batch on
 schedules shortened in proportion.
 """
+import functools
+import hashlib
 import json
 import os
 
 import numpy as np
+
+from . import _lib
 
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "piqmc", "tune.json")
 BLOCKS = (64, 128, 256, 512, 1024)
@@ -59,10 +64,16 @@ def _arch():
     return getattr(p, "gcnArchName", p.name)
 
 
+@functools.lru_cache(maxsize=None)
+def _build(path):
+    with open(path, "rb") as f:
+        return hashlib.sha1(f.read()).hexdigest()[:12]
+
+
 def key(pb, P, R):
     path = 1 if pb.pm_j else (2 if pb.pm_j_fields else 0)
-    return "%s|N%d|Z%d|zmax%d|pmj%d|nc%d|ex%d|P%d|R%d" % (_arch(), pb.nspins, pb.maxnb, pb.zmax,
-                                                          path, pb.ncolors, int(pb.exact_rows), P, R)
+    return "%s|lib%s|N%d|Z%d|zmax%d|pmj%d|nc%d|ex%d|P%d|R%d" % (_arch(), _build(_lib.LIB_PATH), pb.nspins, pb.maxnb,
+                                                                pb.zmax, path, pb.ncolors, int(pb.exact_rows), P, R)
 
 
 def is_dense(pb):
@@ -79,7 +90,9 @@ def candidates(pb, P, R):
             W = P // 2
             if W <= 16 and 16 % W == 0:
                 out += [(b, "split") for b in (64, 128, 256) if b // 64 <= max(1, R)]
-            out += [(256, "workgroup"), (256, "pipe4"), (512, "pipe8"), (64, "fields"), (256, "fields")]
+            out += [(256, "workgroup"), (256, "pipe4"), (512, "pipe8"), (256, "fields")]
+            if pb.nspins > 256:      # (up to there the blocked sweep, which has a workgroup size of its own)
+                out += [(64, "fields")]
         return out
     word = 4 if P // 2 <= 32 else 8
     out = []
@@ -147,8 +160,8 @@ def batch_key(batch):
     shapes = sorted("%d/%d/%d/%d/%d/%d/%d" % (j["problem"].nspins, j["problem"].maxnb,
                                              int(j["problem"].pm_j), j["problem"].ncolors, j["P"], j["R"],
                                              len(j["sched"])) for j in batch.jobs)
-    import hashlib
-    return "%s|batch|%s" % (_arch(), hashlib.sha1("|".join(shapes).encode()).hexdigest()[:16])
+    return "%s|lib%s|batch|%s" % (_arch(), _build(_lib.LIB_PATH),
+                                  hashlib.sha1("|".join(shapes).encode()).hexdigest()[:16])
 
 
 def tune_batch(batch, rpws=(1, 2, 4), shorten=32, use_cache=True, verbose=False):
