@@ -646,7 +646,7 @@ __device__ __forceinline__ float adam_one(const Adam &h, float w, float *m, floa
     return w - h.lr * (mv / h.c1) / (sqrtf(vv / h.c2) + h.eps);
 }
 
-// Adam step on fp32 master weights (masked), refresh bf16 W [O][ldw] and W^T [I][ldt].
+// Adam step on fp32 master weights (masked), refresh bf16 W [O][ldw] and W^T [I][ldt] (null: not kept).
 __global__ void adam_w(float *w, float *m, float *v, const float *g, const uint8_t *mask, int O, int I, Adam h,
                        uint16_t *wb, int ldw, uint16_t *wt, int ldt)
 {
@@ -657,7 +657,7 @@ __global__ void adam_w(float *w, float *m, float *v, const float *g, const uint8
         const uint16_t bb = f2bf_bits(wv);
         const int o = (int)(t / I), i = (int)(t % I);
         wb[(size_t)o * ldw + i] = bb;
-        wt[(size_t)i * ldt + o] = bb;
+        if (wt) wt[(size_t)i * ldt + o] = bb;
     }
 }
 
@@ -1010,14 +1010,15 @@ extern "C" int piqmc_made_create(int N, int H1, int H2, uint64_t seed, piqmc_mad
         hipError_t e = hipSuccess;
         auto A = [&](void **p, size_t bytes) { if (e == hipSuccess) e = hipMalloc(p, bytes); };
         A((void **)&m->w[l], 4 * nw); A((void **)&m->mw[l], 4 * nw); A((void **)&m->vw[l], 4 * nw);
-        A((void **)&m->gw[l], 4 * nw); A((void **)&m->wb[l], 2 * nwb); A((void **)&m->wt[l], 2 * nwt);
+        A((void **)&m->gw[l], 4 * nw); A((void **)&m->wb[l], 2 * nwb);
+        if (l) A((void **)&m->wt[l], 2 * nwt);  // no product takes the input layer's
         A((void **)&m->mask[l], nw); A((void **)&m->b[l], 4 * O); A((void **)&m->mb[l], 4 * O);
         A((void **)&m->vb[l], 4 * O); A((void **)&m->gb[l], 4 * O);
         if (e == hipSuccess) e = hipMemcpy(m->w[l], wv.data(), 4 * nw, hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(m->mask[l], mk.data(), nw, hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemset(m->mw[l], 0, 4 * nw);
         if (e == hipSuccess) e = hipMemset(m->wb[l], 0, 2 * nwb);
-        if (e == hipSuccess) e = hipMemset(m->wt[l], 0, 2 * nwt);
+        if (e == hipSuccess && l) e = hipMemset(m->wt[l], 0, 2 * nwt);
         if (e == hipSuccess) e = hipMemset(m->vw[l], 0, 4 * nw);
         if (e == hipSuccess) e = hipMemset(m->gw[l], 0, 4 * nw);
         if (e == hipSuccess) e = hipMemset(m->b[l], 0, 4 * O);
@@ -1209,7 +1210,7 @@ int train_core(piqmc_made *m, int B, const int8_t *s, const int32_t *perm, int b
                 g.step = lr > 0.f;
                 g.w = m->w[l]; g.m = m->mw[l]; g.v = m->vw[l]; g.mask = m->mask[l];
                 g.Cb = m->wb[l]; g.ldc = up64(g.N);
-                g.Ct = l ? m->wt[l] : nullptr; g.ldt = up64(g.M);  // the input layer's transpose is not used
+                g.Ct = m->wt[l]; g.ldt = up64(g.M);
                 g.gt = gt[l]; g.ldg = lB; g.units = g.M; g.rows = B; g.n64 = (g.M + 63) / 64;
                 g.gb = m->gb[l]; g.b = m->b[l]; g.bm = m->mb[l]; g.bv = m->vb[l];
                 jobs.blocks[jobs.n] = g.n64 + tiles_of(g.M, g.N);

@@ -10,7 +10,7 @@ struct piqmc_made {
     int padded = 0;  // what lies past the sizes in their rows is zero
     int layers_in[3], layers_out[3];
     float *w[3] = {}, *b[3] = {}, *mw[3] = {}, *vw[3] = {}, *mb[3] = {}, *vb[3] = {};
-    uint16_t *wb[3] = {}, *wt[3] = {};   // bf16 [out][in], [in][out], row pitches rounded up to 64, zeros past the sizes
+    uint16_t *wb[3] = {}, *wt[3] = {};   // bf16 [out][in], [in][out] (not the first), row pitches rounded up to 64, zeros past the sizes
     uint8_t *mask[3] = {};
     float *gw[3] = {}, *gb[3] = {};
     // activations [cap][*] and their gradients [tcap][*], row pitches (but the logits') rounded up to 64

@@ -58,12 +58,10 @@ constexpr int kCap = 128;                    // queue entries per wavefront (at 
 
 template <typename WT>
 struct SparseArgs {
-    int N, P, W, S, M, ncolors, R, rpw, Z;
+    int N, P, W, S, M, ncolors, R, rpw;
     uint32_t key0, key1, replica_base, sweep_base;
     const float *jperp, *temps;   // [S]
     const int *color_off;         // [ncolors + 1]
-    const int32_t *order;         // [N]
-    const int2 *rows;             // [N][Z] (energies)
     piqmc::SparseTab t;
     WT *packed;                   // [R][2][N]
     double *etrace;               // [R][S] or null
@@ -486,10 +484,10 @@ SparseArgs<WT> args_of(const piqmc::SparseCall &c)
     const piqmc_problem *pb = c.pb;
     SparseArgs<WT> a;
     a.N = pb->N; a.P = c.P; a.W = c.P / 2; a.S = c.S; a.M = c.M; a.ncolors = pb->ncolors; a.R = c.R;
-    a.rpw = c.rpw; a.Z = pb->Z;
+    a.rpw = c.rpw;
     a.key0 = (uint32_t)c.seed; a.key1 = (uint32_t)(c.seed >> 32);
     a.replica_base = c.rbase; a.sweep_base = c.sbase;
-    a.jperp = c.jperp; a.temps = c.temps; a.color_off = c.color_off; a.order = pb->d_order; a.rows = pb->d_rows;
+    a.jperp = c.jperp; a.temps = c.temps; a.color_off = c.color_off;
     a.t = pb->sparse;
     a.packed = reinterpret_cast<WT *>(c.packed);
     a.etrace = c.etrace;
