@@ -6,7 +6,7 @@
 // row times the time of one.  With the local fields cached in LDS a decision
 // still took about 1100 cycles -- an LDS read, a division and an exponential,
 // two or more Philox blocks, an LDS update of the row -- and a sweep had 2 N of
-// them.  Here a sweep has N, of 100-odd cycles each:
+// them.  Here a sweep has N, of about 430 cycles each:
 //   - Draws ahead.  A uniform u does not depend on the state, so the test
 //     exp(ediff / T) > u is turned into ediff > T ln(u) and the threshold is
 //     ready before the decision: idle wavefronts draw the next block's Philox
@@ -26,10 +26,10 @@
 //   - Both parities at once.  Two teams, one a parity, the odd one a block
 //     behind: it reads the even parity's spins only in the block it is in, which
 //     the even team has left and comes back to a whole sweep later.
-// Per position of both parities, 256 spins, against the cached-field sweep over
-// eight wavefronts: P=16 1013 -> 171 ns, P=32 1042 -> 214 ns, P=128 1409 -> 568 ns;
-// 1024 replicas of P=32 4294 -> 1404 ns, of P=128 9103 -> 5770 ns.  At P=32 a block
-// takes 7000 cycles: 3200 to decide (16 chains of five dependent instructions,
+// Per position of both parities, 256 spins, 4 replicas, against the cached-field
+// sweep over eight wavefronts: P=16 1013 -> 169 ns, P=32 1042 -> 178 ns, P=128 1409
+// -> 345 ns; 1024 replicas of P=32 4294 -> 730 ns, of P=128 9103 -> 1398 ns.  At P=32 a
+// block takes 7000 cycles: 3200 to decide (16 chains of five dependent instructions,
 // an LDS read of couplings each), about as long beside it for the draws, 3000 to
 // apply its few flips and hand over, the rest at the two barriers.
 #include <math.h>
@@ -314,8 +314,11 @@ __device__ void block_sweep(const BlockArgs &a, int r, unsigned char *smem)
                 const bool act = ln < W;
                 const int lb = act ? ln : 0;
                 // open below this distance from the threshold: the logarithm's
-                // error (2e-5 of up to 11.5 T, a wide margin) and 17 roundings of
-                // sums below bound plus the field itself
+                // error (2e-5 of up to 11.5 T, a wide margin) and the roundings of the
+                // field and of the 16 sums after it.  The field is at most bound; a sum
+                // that ends near its threshold has J_perp ts within bound + 11.5 T, so
+                // none exceeds 2 bound + 11.5 T: 33 half units of the last place of
+                // bound, 1.97e-6, and 1.2e-5 T, which the logarithm's margin holds
                 const float gd = 2.5e-4f * T + 2e-6f * a.bound;
                 const float *tb = th + buf * kB * WP;
                 const f4 *J = reinterpret_cast<const f4 *>(jb + buf * kB * kB);
