@@ -58,10 +58,14 @@ constexpr int kCap = 128;                    // queue entries per wavefront (at 
 
 template <typename WT>
 struct SparseArgs {
-    int N, P, W, S, M, ncolors, R, rpw;
+    int N, P, W, S, M, ncolors, R, rpw, pad0;
     uint32_t key0, key1, replica_base, sweep_base;
     const float *jperp, *temps;   // [S]
     const int *color_off;         // [ncolors + 1]
+    // room only: the tables at byte 96 and J_perp at 56 is what the argument loads
+    // do best with (without: 10^3, P=64, 128 replicas 440 -> 446 us; 16 x 16, P=128, 512
+    // 311 -> 322; 80 x 80, P=20, 32 1816 -> 1842)
+    const void *pad1[2];
     piqmc::SparseTab t;
     WT *packed;                   // [R][2][N]
     double *etrace;               // [R][S] or null
