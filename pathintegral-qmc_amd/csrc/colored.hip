@@ -2797,8 +2797,8 @@ int default_block(const piqmc_problem *pb, int R, int rpw, int word_bytes, bool 
         // 600 replicas 170 us at 512, 208 at 1024; 14^3, 1372, P=64, 600: 208 / 237; 56
         // x 56, 1568, P=20, 600: 244 / 227; 46 x 46, 2048 replicas, four a workgroup:
         // 384 / 295; 10 steps each); with a workgroup a CU its time is all that counts.
-        const bool filled = word_bytes == 8 || biggest > 1536 || rpw >= 4 || (R + rpw - 1) / rpw <= cu_count();
-        if (biggest > 1024 && biggest <= 2048 && filled && queue_lds(pb->N, rpw, word_bytes, 1024) <= 160 * 1024)
+        if (biggest > 1024 && biggest <= 2048 && queue_lds(pb->N, rpw, word_bytes, 1024) <= 160 * 1024 &&
+            (word_bytes == 8 || biggest > 1536 || rpw >= 4 || (R + rpw - 1) / rpw <= cu_count()))
             return 1024;
         return block;
     }
