@@ -276,10 +276,10 @@ static int upload_coloring(piqmc_problem &p)
     }
     PIQMC_HIP(hipMalloc(&p.d_prevj, sizeof(double) * N));
     PIQMC_HIP(hipMemcpy(p.d_prevj, prevj.data(), sizeof(double) * N, hipMemcpyHostToDevice));
-    if (const int rc = piqmc::block_upload(p, order)) return rc;
-    if (!p.pmj && !p.pmjf) {
-        const int rc = piqmc::sparse_upload(p, order);
-        if (rc) return rc;
+    if (p.sweeps) {
+        if (const int rc = piqmc::block_upload(p, order)) return rc;
+        if (!p.pmj && !p.pmjf)
+            if (const int rc = piqmc::sparse_upload(p, order)) return rc;
     }
     if (p.pmj || p.pmjf) {
         const int zm = std::max(p.zmax, 1);
@@ -314,12 +314,13 @@ static int upload_coloring(piqmc_problem &p)
     return PIQMC_OK;
 }
 
-extern "C" int piqmc_problem_create(int N, int Z, const double *nbs, piqmc_problem **out)
+int piqmc::problem_create(int N, int Z, const double *nbs, bool sweeps, piqmc_problem **out)
 {
     if (!out) return set_error(PIQMC_EINVAL, "null output handle");
     *out = nullptr;
     if (N < 1 || Z < 1 || !nbs) return set_error(PIQMC_EINVAL, "nspins and maxnb must be >= 1");
     auto *p = new piqmc_problem();
+    p->sweeps = sweeps;
     p->N = N;
     p->Z = Z;
     p->idx.resize((size_t)N * Z);
@@ -448,8 +449,7 @@ extern "C" int piqmc_problem_create(int N, int Z, const double *nbs, piqmc_probl
 // lower triangle is never read).  A zero coupling adds +-0 to the running
 // float ediff, which changes neither its value nor any later comparison, so
 // zero entries are dropped and the surviving terms keep their order.
-extern "C" int piqmc_problem_create_dense(int N, const double *Jm, int64_t s0, int64_t s1,
-                                          piqmc_problem **out)
+int piqmc::problem_create_dense(int N, const double *Jm, int64_t s0, int64_t s1, bool sweeps, piqmc_problem **out)
 {
     if (!out) return set_error(PIQMC_EINVAL, "null output handle");
     *out = nullptr;
@@ -475,7 +475,7 @@ extern "C" int piqmc_problem_create_dense(int N, const double *Jm, int64_t s0, i
             jd[(size_t)i * Z + e] = rows[i][e].second;
         }
     piqmc_problem *p = nullptr;
-    int rc = piqmc_problem_create(N, Z, nbs.data(), &p);
+    int rc = piqmc::problem_create(N, Z, nbs.data(), sweeps, &p);
     if (rc) return rc;
     p->dense = 1;
     hipError_t e = hipMalloc(&p->d_jd, sizeof(double) * jd.size());
@@ -486,6 +486,16 @@ extern "C" int piqmc_problem_create_dense(int N, const double *Jm, int64_t s0, i
     }
     *out = p;
     return PIQMC_OK;
+}
+
+extern "C" int piqmc_problem_create(int N, int Z, const double *nbs, piqmc_problem **out)
+{
+    return piqmc::problem_create(N, Z, nbs, true, out);
+}
+
+extern "C" int piqmc_problem_create_dense(int N, const double *Jm, int64_t s0, int64_t s1, piqmc_problem **out)
+{
+    return piqmc::problem_create_dense(N, Jm, s0, s1, true, out);
 }
 
 extern "C" int piqmc_problem_destroy(piqmc_problem *p)

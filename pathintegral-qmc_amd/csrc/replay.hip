@@ -859,8 +859,8 @@ int dropin(const double *sched, int S, int M, int P, float temp, int N, double *
             p16[g * N + t] = (uint16_t)v;
         }
     piqmc_problem *pb = nullptr;
-    int rc = cp.J ? piqmc_problem_create_dense(N, cp.J, cp.js0, cp.js1, &pb)
-                  : piqmc_problem_create(N, cp.Z, cp.nbs, &pb);
+    int rc = cp.J ? piqmc::problem_create_dense(N, cp.J, cp.js0, cp.js1, false, &pb)
+                  : piqmc::problem_create(N, cp.Z, cp.nbs, false, &pb);
     if (rc) return rc;
     struct Guard {
         piqmc_problem *p;
