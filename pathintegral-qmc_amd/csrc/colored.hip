@@ -2673,8 +2673,8 @@ struct CallBuffers {
 
 // The host tables of a call, uploaded as one buffer by one copy: each further
 // allocation and copy of a small call costs the host more than the tables' bytes
-// (64 spins, one replica, 100 steps: 426 us with a copy each, 417 so).  Each table
-// begins at a multiple of 256 bytes.
+// (64 spins, one replica, 100 steps: 425 us with a copy each, 414 so, where two
+// runs of either differ by 2 %).  Each table begins at a multiple of 256 bytes.
 struct Table {
     const void *src;  // null: room only
     size_t bytes;

@@ -6,7 +6,7 @@
 // row times the time of one.  With the local fields cached in LDS a decision
 // still took about 1100 cycles -- an LDS read, a division and an exponential,
 // two or more Philox blocks, an LDS update of the row -- and a sweep had 2 N of
-// them.  Here a sweep has N, of about 430 cycles each:
+// them.  Here a sweep has N, of about 410 cycles each:
 //   - Draws ahead.  A uniform u does not depend on the state, so the test
 //     exp(ediff / T) > u is turned into ediff > T ln(u) and the threshold is
 //     ready before the decision: idle wavefronts draw the next block's Philox
@@ -29,7 +29,7 @@
 // Per position of both parities, 256 spins, 4 replicas, against the cached-field
 // sweep over eight wavefronts: P=16 1013 -> 169 ns, P=32 1042 -> 178 ns, P=128 1409
 // -> 345 ns; 1024 replicas of P=32 4294 -> 730 ns, of P=128 9103 -> 1398 ns.  At P=32 a
-// block takes 7000 cycles: 3200 to decide (16 chains of five dependent instructions,
+// block takes 6600 cycles: 3200 to decide (16 chains of five dependent instructions,
 // an LDS read of couplings each), about as long beside it for the draws, 3000 to
 // apply its few flips and hand over, the rest at the two barriers.
 #include <math.h>

@@ -38,8 +38,9 @@
 // replicas, 30 traced steps 10.35 -> 0.58 ms; 80 x 80 Gaussian lattice, P=20,
 // T=0.01, 32 replicas, 40 steps 18.6 -> 1.93 ms, and its 32 classical chains
 // over 40 temperatures 18.6 -> 0.51 ms (32 workgroups instead of one).  Bound by
-// VALU issue (77 % of the cycles of the CUs in use, 445 instructions per 64
-// words on the 80 x 80 lattice).
+// VALU issue (77 % of the cycles of the CUs in use, 450 instructions per 64
+// words on the 80 x 80 lattice; 64 % and 951 on the 10^3, whose wavefronts end
+// every slot with a partly filled drain).
 #include <math.h>
 
 #include <algorithm>
