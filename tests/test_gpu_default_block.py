@@ -46,15 +46,13 @@ def _near_the_best(gpu, L, dim, P, R, blocks):
     c8 = torch.ones((R, P, N), dtype=torch.int8, device=gpu)
     sched = np.linspace(3.0, 1e-8, 20)
 
-    def ms(block):
-        best = np.inf
-        for _ in range(6):
+    best = dict.fromkeys((0,) + blocks, np.inf)
+    for _ in range(6):                   # in turn, the first round to warm up
+        for block in best:
             c8.fill_(1)
             pb.qa_colored(c8, sched, 1, 1.0 / P, 5, block=block)
-            best = min(best, device.last_kernel_ms())
-        return best
-
-    assert ms(0) <= 1.1 * min(ms(b) for b in blocks)
+            best[block] = min(best[block], device.last_kernel_ms())
+    assert best.pop(0) <= 1.1 * min(best.values())
 
 
 @pytest.mark.parametrize("L,dim,P,R", [(46, 2, 20, 600), (14, 3, 20, 1000), (46, 2, 64, 100), (46, 2, 128, 600),

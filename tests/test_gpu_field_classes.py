@@ -105,14 +105,11 @@ def test_default_tile_is_near_the_best(gpu, L, dim, P, R):
     c8 = torch.ones((R, P, N), dtype=torch.int8, device=gpu)
     sched = np.linspace(3.0, 1e-8, 6)
 
-    def ms(rpw):
-        best = np.inf
-        for _ in range(5):
+    word = 4 if P <= 64 else 8
+    best = dict.fromkeys([0] + [r for r in (1, 2, 3, 4, 6, 8, 12, 16) if 2 * N * word * r < 150000], np.inf)
+    for _ in range(5):                   # in turn, the first round to warm up
+        for rpw in best:
             c8.fill_(1)
             pb.qa_colored(c8, sched, 1, 1.0 / P, 5, rpw=rpw)
-            best = min(best, device.last_kernel_ms())
-        return best
-
-    word = 4 if P <= 64 else 8
-    fits = [r for r in (1, 2, 3, 4, 6, 8, 12, 16) if 2 * N * word * r < 150000]
-    assert ms(0) <= 1.2 * min(ms(r) for r in fits)
+            best[rpw] = min(best[rpw], device.last_kernel_ms())
+    assert best.pop(0) <= 1.2 * min(best.values())
